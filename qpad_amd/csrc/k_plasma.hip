@@ -3,13 +3,12 @@
 // current/acceleration/momentum-flux deposit, and the fused push_u + push_x.
 //
 // Particles are kept sorted by radial cell (cell c = int(r/dr), nodes c+1 and
-// c+2).  Deposits run one wavefront per chunk of at most kDepChunk particles
-// of a cell: each lane accumulates its particles in registers, the wavefront
-// reduces with a fixed butterfly and writes the chunk's partials for node c+1
-// (P0) and node c+2 (P1) once.  A cell's first chunk goes to P0/P1[c], its
-// further chunks (crowded cells only) to the overflow rows O0/O1 the sort
-// lists; the field kernels add P0[i-1] + P1[i-2] per node, each with its
-// cell's overflow rows in row order.  No atomics, deterministic order.
+// c+2).  A wavefront deposits a cell of ordinary size; the chunks (at most
+// kDepChunk particles) of a crowded cell are each deposited by four
+// wavefronts.  The partials of a cell's first chunk for node c+1 and node c+2
+// go to P0/P1[c], those of its further chunks to the overflow rows O0/O1 the
+// sort numbers; the field kernels add P0[i-1] + P1[i-2] per node, each with
+// its cell's overflow rows in row order.  No atomics, deterministic order.
 #include <algorithm>
 #include <cstring>
 
@@ -234,67 +233,78 @@ struct QDepArgs {
     double qbm;
     const int32_t *cs;
     double *P0, *P1;
-    // overflow chunks (listed by the sort) and their partial rows
+    // the crowded cells' chunks (listed by the sort) and the overflow rows
     const int32_t *os;
     const int4 *desc;
     double *O0, *O1;
-    int n_ov_max;
+    int first, n_crowd_max;
 };
 
-// One wave per chunk of at most kDepChunk particles of one cell.  The first
-// ceil(nr / CPW) workgroups take the first chunk of cell (workgroup * CPW +
-// wave) into P0/P1; the workgroups after them take the overflow chunks
-// (row = (workgroup - ceil(nr / CPW)) * CPW + wave) into O0/O1.
-// CPW: waves per workgroup, a launch shape the tuner chooses
-// (qpad_tune_launch); every wave's work and result are the same for every
-// shape.
-struct DepChunk {
-    int cell, pb, pe, row;
-    bool ovf, live;
-};
+// What a deposit workgroup of CPW waves does.  The first ceil(nr / CPW)
+// workgroups take the cells of at most `first` particles, one wave per cell
+// (cell = workgroup * CPW + wave), into P0/P1.  The workgroups after them
+// walk the list of crowded chunks: every chunk is cut into kDepSub parts of
+// kDepChunk / kDepSub particles, one wave per part (a wave takes two parts
+// where CPW = 2, a workgroup two chunks where CPW = 8), whose sums are added
+// in LDS in part order into the chunk's row.  A single wave over a whole
+// chunk (16 passes) would hold the launch up long after the ordinary cells
+// are done.  CPW: waves per workgroup, a launch shape the tuner chooses
+// (qpad_tune_launch); every part's work and the order of the sums are the
+// same for every shape.
+constexpr int kDepSub = 4;
+constexpr int kDepPart = kDepChunk / kDepSub;
+// at most this many workgroups walk the crowded list
+constexpr int kCrowdGroups = 256;
 
 template <int CPW>
-__device__ __forceinline__ DepChunk dep_chunk(int nr, const int32_t *cs, const int32_t *os, const int4 *desc,
-                                              int n_ov_max, int wave)
+constexpr int crowd_chunks() { return CPW >= 2 * kDepSub ? CPW / kDepSub : 1; }   // chunks of a workgroup at once
+template <int CPW>
+constexpr int crowd_parts() { return CPW < kDepSub ? kDepSub / CPW : 1; }         // parts of a wave
+
+struct DepRange {
+    int cell, pb, pe;
+};
+
+// the cell of a wave (cells of more than `first` particles are on the
+// crowded list; live false for those and past the last cell)
+template <int CPW>
+__device__ __forceinline__ DepRange cell_range(int nr, const int32_t *cs, int first, int wave, bool &live)
 {
-    DepChunk k;
-    const int ncg = (nr + CPW - 1) / CPW;
-    k.ovf = (int)blockIdx.x >= ncg;
-    if (!k.ovf) {
-        const int c = blockIdx.x * CPW + wave;
-        k.live = c < nr;
-        k.cell = min(c, nr - 1);
-        k.row = k.cell;
-        const int p0 = cs[k.cell], p1 = cs[k.cell + 1];
-        k.pb = p0;
-        k.pe = min(p1, p0 + kDepChunk);
-    } else {
-        const int o = ((int)blockIdx.x - ncg) * CPW + wave;
-        const int nov = os[nr];
-        const int4 d = desc[min(o, n_ov_max - 1)];
-        k.live = o < nov;
-        k.cell = min(max(d.x, 0), nr - 1);
-        k.row = min(o, n_ov_max - 1);
-        k.pb = d.y;
-        k.pe = k.live ? d.z : d.y;
-    }
+    const int c = blockIdx.x * CPW + wave;
+    DepRange k;
+    k.cell = min(c, nr - 1);
+    k.pb = __builtin_amdgcn_readfirstlane(cs[k.cell]);
+    k.pe = __builtin_amdgcn_readfirstlane(cs[k.cell + 1]);
+    live = c < nr && k.pe - k.pb <= first;
     return k;
 }
 
-// overflow workgroups none of whose waves has a chunk (the grid is sized
-// for the most chunks the particle count allows); uniform over the workgroup
-template <int CPW>
-__device__ __forceinline__ bool dep_group_idle(int nr, const int32_t *os)
+// entry o of the crowded list (uniform over the wave)
+__device__ __forceinline__ int4 crowd_entry(const int4 *desc, int o)
 {
-    const int ncg = (nr + CPW - 1) / CPW;
-    return (int)blockIdx.x >= ncg && ((int)blockIdx.x - ncg) * CPW >= os[nr];
+    const int4 d = desc[o];
+    return make_int4(__builtin_amdgcn_readfirstlane(d.x), __builtin_amdgcn_readfirstlane(d.y),
+                     __builtin_amdgcn_readfirstlane(d.z), __builtin_amdgcn_readfirstlane(d.w));
 }
 
-// overflow rows the grid provides for (at most) npp particles in the box
-inline int dep_grid(int nr, int64_t npp, int n_ov_max, int cpw)
+// part `sub` of a crowded chunk (cell, first particle, end, row)
+__device__ __forceinline__ DepRange part_range(const int4 &d, int sub, bool live)
 {
-    const int nov = (int)std::min<int64_t>(npp / kDepChunk + 1, n_ov_max);
-    return (nr + cpw - 1) / cpw + (nov + cpw - 1) / cpw;
+    DepRange k;
+    k.cell = d.x;
+    k.pb = min(d.y + sub * kDepPart, d.z);
+    k.pe = live ? min(k.pb + kDepPart, d.z) : k.pb;
+    return k;
+}
+
+// workgroups of a deposit over (at most) npp particles: the cells', then the
+// crowded list's (a chunk holds kDepChunk particles or closes a cell of more
+// than `first`)
+inline int dep_grid(int nr, int64_t npp, int first, int cpw)
+{
+    const int chunks = (int)std::min<int64_t>(npp / (first + 1) + npp / kDepChunk, 1 << 20);
+    const int per = cpw >= 2 * kDepSub ? cpw / kDepSub : 1;
+    return (nr + cpw - 1) / cpw + std::min((chunks + per - 1) / per, kCrowdGroups);
 }
 
 // the arguments of every species of one launch (workgroup rows by species)
@@ -302,27 +312,20 @@ struct QDepMulti {
     QDepArgs s[kMaxSpecies];
 };
 
+// sums of the particles [p0, p1) of cell c over the wave: lane l ends with
+// values [(l / 4) NB, (l / 4 + 1) NB) of [node][mode array] (padded to 16 NB)
 // CHI: deposit_chi_part2d (part2d_class.f03:361-476) instead: each particle
 // deposits -(q/m) q / (1 - (q/m) psi) in place of q
-template <int M, int CPW, bool CHI = false>
-__global__ __launch_bounds__(64 * CPW) void k_qdeposit(const QDepMulti m)
+template <int M, bool CHI, int NB>
+__device__ __forceinline__ void qdep_sums(const QDepArgs &a, int c, int p0, int p1, int lane, double (&acc)[16 * NB])
 {
-    const QDepArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     constexpr int NM = 2 * M + 1;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const DepChunk ch = dep_chunk<CPW>(a.nr, a.cs, a.os, a.desc, a.n_ov_max, wave);
-    if (!ch.live) return;
-    const int c = ch.cell, p0 = ch.pb, p1 = ch.pe;
-    // acc[k]: node ix, acc[NM + k]: node ix + 1; padded to a multiple of 16
-    constexpr int NB = (2 * NM + 15) / 16;
-    double acc[16 * NB];
 #pragma unroll
     for (int v = 0; v < 16 * NB; v++) acc[v] = 0.0;
     // wave-uniform passes, software-pipelined as in k_amjdeposit; lanes past
-    // the chunk's end deposit zero
+    // the range's end deposit zero
     const int npass = __builtin_amdgcn_readfirstlane((p1 - p0 + 63) >> 6);
-    const int pl = max(p1 - 1, p0);
+    const int pl = max(p1 - 1, 0);
     int p = p0 + lane;
     int pc = min(p, pl);
     double nx1 = a.x1[pc], nx2 = a.x2[pc], nq = a.q[pc];
@@ -354,15 +357,60 @@ __global__ __launch_bounds__(64 * CPW) void k_qdeposit(const QDepMulti m)
         }
     }
     wave_reduce_scatter<NB>(acc);
-    const int g = lane >> 2;
-    double *D0 = ch.ovf ? a.O0 : a.P0, *D1 = ch.ovf ? a.O1 : a.P1;
+}
+
+template <int M, int CPW, bool CHI = false>
+__global__ __launch_bounds__(64 * CPW) void k_qdeposit(const QDepMulti m)
+{
+    const QDepArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
+    constexpr int NM = 2 * M + 1, NB = (2 * NM + 15) / 16;
+    constexpr int CH = crowd_chunks<CPW>(), PT = crowd_parts<CPW>();
+    __shared__ double comb[CH][kDepSub][2 * NM];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ncg = (a.nr + CPW - 1) / CPW;
+    double acc[16 * NB];
+    // value v of this lane's sums to D0[v] (node ix) or D1[v - NM] (node ix + 1)
+    auto store = [&](double *D0, double *D1) {
 #pragma unroll
-    for (int i = 0; i < NB; i++) {
-        const int v = g * NB + i;
-        if ((lane & 3) == (i & 3) && v < 2 * NM) {
-            if (v < NM) D0[(size_t)ch.row * NM + v] = acc[i];
-            else D1[(size_t)ch.row * NM + v - NM] = acc[i];
+        for (int i = 0; i < NB; i++) {
+            const int v = (lane >> 2) * NB + i;
+            if ((lane & 3) == (i & 3) && v < 2 * NM) {
+                if (v < NM) D0[v] = acc[i];
+                else D1[v - NM] = acc[i];
+            }
         }
+    };
+    if ((int)blockIdx.x < ncg) {
+        bool live;
+        const DepRange r = cell_range<CPW>(a.nr, a.cs, a.first, wave, live);
+        if (!live) return;
+        qdep_sums<M, CHI, NB>(a, r.cell, r.pb, r.pe, lane, acc);
+        store(a.P0 + (size_t)r.cell * NM, a.P1 + (size_t)r.cell * NM);
+        return;
+    }
+    const int n = min(a.os[a.nr + 1], a.n_crowd_max), step = ((int)gridDim.x - ncg) * CH;
+    for (int o0 = ((int)blockIdx.x - ncg) * CH; o0 < n; o0 += step) {
+        const int ch = wave / (CPW / CH), o = o0 + ch;
+        const bool live = o < n;
+        const int4 d = crowd_entry(a.desc, min(o, n - 1));
+#pragma unroll
+        for (int u = 0; u < PT; u++) {
+            const int sub = (wave % (CPW / CH)) * PT + u;
+            const DepRange r = part_range(d, sub, live);
+            qdep_sums<M, CHI, NB>(a, r.cell, r.pb, r.pe, lane, acc);
+            store(comb[ch][sub], comb[ch][sub] + NM);
+        }
+        __syncthreads();
+        for (int t = threadIdx.x; t < CH * 2 * NM; t += 64 * CPW) {
+            const int q = t / (2 * NM), v = t % (2 * NM);
+            if (o0 + q >= n) continue;
+            const int4 e = a.desc[o0 + q];
+            const double sum = ((comb[q][0][v] + comb[q][1][v]) + comb[q][2][v]) + comb[q][3][v];
+            double *D = e.w < 0 ? (v < NM ? a.P0 : a.P1) + (size_t)e.x * NM : (v < NM ? a.O0 : a.O1) + (size_t)e.w * NM;
+            D[v < NM ? v : v - NM] = sum;
+        }
+        __syncthreads();
     }
 }
 
@@ -382,7 +430,8 @@ static QDepArgs qdep_args(qpad_ctx *c, int s)
     a.desc = sp.ov_desc;
     a.O0 = sp.O0;
     a.O1 = sp.O1;
-    a.n_ov_max = sp.n_ov_max;
+    a.first = sp.dep_first;
+    a.n_crowd_max = sp.n_crowd_max;
     return a;
 }
 
@@ -428,7 +477,7 @@ int launch_qdeposit_range(qpad_ctx *c, int s0, int s1)
     int gx = 1;
     for (int s = s0; s < s1; s++) {
         m.s[s - s0] = qdep_args(c, s);
-        gx = std::max(gx, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].n_ov_max, c->dep_cells));
+        gx = std::max(gx, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].dep_first, c->dep_cells));
     }
     return qdeposit_launch(c, m, s1 - s0, gx);
 }
@@ -446,7 +495,7 @@ int launch_qdeposit_rows(qpad_ctx *c, int s, const DepRows &rows)
     m.s[0].P1 = rows.P1;
     m.s[0].O0 = rows.O0;
     m.s[0].O1 = rows.O1;
-    const int gx = std::max(1, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].n_ov_max, c->dep_cells));
+    const int gx = std::max(1, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].dep_first, c->dep_cells));
     return qdeposit_launch(c, m, 1, gx);
 }
 
@@ -461,7 +510,7 @@ int launch_chi_deposit_rows(qpad_ctx *c, int s, const DepRows &rows)
     m.s[0].P1 = rows.P1;
     m.s[0].O0 = rows.O0;
     m.s[0].O1 = rows.O1;
-    const int gx = std::max(1, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].n_ov_max, c->dep_cells));
+    const int gx = std::max(1, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].dep_first, c->dep_cells));
     return qdeposit_launch(c, m, 1, gx, true);
 }
 
@@ -534,6 +583,54 @@ __device__ __forceinline__ void gather3(const F &f, double w0, double w1, double
     gather_n<M, 3>(f, w0, w1, pc, ps, out);
 }
 
+// E and B at a particle from the packed fields eb[node][k][e_r, e_phi, e_z,
+// b_r, b_phi, b_z] (qpad_ctx::eb), p at node ix: the six sums over (node,
+// mode array) of the field times w_n times the mode's cos or -sin (doubled
+// above m = 0).  `fence` runs before each node's loads of a mode.
+template <int M, class P, class F>
+__device__ __forceinline__ void gather_eb(P p, double w0, double w1, double pc, double ps, double ep[3], double bp[3],
+                                          const F &fence)
+{
+    constexpr int N1 = 6 * (2 * M + 1);   // one node's values
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        ep[c] = p[c] * w0 + p[N1 + c] * w1;
+        bp[c] = p[3 + c] * w0 + p[N1 + 3 + c] * w1;
+    }
+    double phr = 1.0, phi = 0.0;
+#pragma unroll
+    for (int m = 1; m <= M; m++) {
+        const double tr = phr * pc - phi * ps, ti = phr * ps + phi * pc;
+        phr = tr;
+        phi = ti;
+        const double re = 2.0 * phr, im = -2.0 * phi;
+        const int kr = 6 * (2 * m - 1), ki = 6 * (2 * m);
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            const double rn = re * (n ? w1 : w0), in = im * (n ? w1 : w0);
+            fence(p);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                ep[c] = ep[c] + p[n * N1 + kr + c] * rn + p[n * N1 + ki + c] * in;
+                bp[c] = bp[c] + p[n * N1 + kr + 3 + c] * rn + p[n * N1 + ki + 3 + c] * in;
+            }
+        }
+    }
+}
+
+// the packed fields through the scalar cache: a wave that works on one cell
+// reads its two nodes into SGPRs (one operand of every gather FMA), which
+// leaves the LDS and its bandwidth to the products
+typedef const double __attribute__((address_space(4))) *uniform_ptr;
+
+// keeps one node's values of a mode in SGPRs at a time (all would not fit)
+struct UniformFence {
+    __device__ __forceinline__ void operator()(uniform_ptr &p) const { __asm__ volatile("" : "+s"(p)); }
+};
+struct NoFence {
+    __device__ __forceinline__ void operator()(const double *) const {}
+};
+
 // nodes ix, ix + 1 of a slice field in HBM
 struct NodePair {
     const double *f;
@@ -583,7 +680,7 @@ struct JDepArgs {
     double *gamma, *psi;
     int store_diag;
     const int32_t *cs;
-    const double *e, *b;
+    const double *eb;   // the packed E and B of the slice (qpad_ctx::eb)
     // the laser envelope and its gradients of the slice (PGC pushers)
     const double *ar, *ai, *arg, *aig;
     double *P0, *P1;
@@ -596,11 +693,11 @@ struct JDepArgs {
     // host-visible copy of the decision (done, iterations so far) written by
     // workgroup 0 of a SPEC launch, or null
     IterState *report;
-    // overflow chunks (listed by the sort) and their partial rows
+    // the crowded cells' chunks (listed by the sort) and the overflow rows
     const int32_t *os;
     const int4 *desc;
     double *O0, *O1;
-    int n_ov_max;
+    int first, n_crowd_max;
 };
 
 // What one particle deposits (robust predictor, part2d_class.f03:877-960):
@@ -616,54 +713,26 @@ struct PartTerms {
     double ph[2 * M + 1];
 };
 
-// the products the reduce-scatter form accumulates: value v is
-// (w[n] ph[k]) val[comp]
-template <int M>
-struct DepTerms {
-    double val[8];
-    double wph[2][2 * M + 1];
-    __device__ __forceinline__ explicit DepTerms(const PartTerms<M> &t)
-    {
-#pragma unroll
-        for (int c = 0; c < 8; c++) val[c] = t.val[c];
-#pragma unroll
-        for (int n = 0; n < 2; n++)
-#pragma unroll
-            for (int k = 0; k < 2 * M + 1; k++) wph[n][k] = t.w[n] * t.ph[k];
-    }
-    __device__ __forceinline__ double operator()(int v) const
-    {
-        constexpr int NM = 2 * M + 1;
-        const int n = v / (8 * NM), r = v % (8 * NM);
-        return wph[n][r % NM] * val[r / NM];
-    }
-};
-
-// the values a deposit workgroup stages in LDS per wave: E, B ([n][cc][k]),
-// then for the PGC pushers ar, ai ([n][k]) and ar_grad, ai_grad ([n][cc][k])
+// the laser values a PGC deposit workgroup stages in LDS per wave: ar, ai
+// ([n][k]) and ar_grad, ai_grad ([n][cc][k])
 template <int NM, bool PGC>
-constexpr int dep_staged() { return PGC ? 28 * NM : 12 * NM; }
+constexpr int dep_staged() { return PGC ? 16 * NM : 1; }
 
-// staged value l of the PGC layout of the cell whose left node is ix
+// staged value l of the cell whose left node is ix
 template <int NM>
-__device__ __forceinline__ double dep_stage_load_pgc(const double *e, const double *b, const double *ar,
-                                                     const double *ai, const double *arg, const double *aig, int nm,
-                                                     int ld, int l, int ix)
+__device__ __forceinline__ double dep_stage_load_pgc(const double *ar, const double *ai, const double *arg,
+                                                     const double *aig, int nm, int ld, int l, int ix)
 {
     const double *f;
     int nc, base;
-    if (l < 12 * NM) {
-        f = l < 6 * NM ? e : b;
-        nc = 3;
-        base = l < 6 * NM ? 0 : 6 * NM;
-    } else if (l < 16 * NM) {
-        f = l < 14 * NM ? ar : ai;
+    if (l < 4 * NM) {
+        f = l < 2 * NM ? ar : ai;
         nc = 1;
-        base = l < 14 * NM ? 12 * NM : 14 * NM;
+        base = l < 2 * NM ? 0 : 2 * NM;
     } else {
-        f = l < 22 * NM ? arg : aig;
+        f = l < 10 * NM ? arg : aig;
         nc = 3;
-        base = l < 22 * NM ? 16 * NM : 22 * NM;
+        base = l < 10 * NM ? 4 * NM : 10 * NM;
     }
     const int r = l - base, n = r / (nc * NM), comp = (r / NM) % nc, k = r % NM;
     return f[((size_t)comp * nm + k) * ld + ix + n];
@@ -679,11 +748,13 @@ __device__ __forceinline__ double dep_stage_load_pgc(const double *e, const doub
 // electric field the ponderomotive term -+ (q/m)/(2 gamma) a grad a
 // (r, phi minus, z plus, with the initial gamma), and the robust form
 // normalises its second half kick by gamma / (gamma - u_z) of the rotated
-// momentum.  sf: the wave's staged values (dep_staged layout).
+// momentum.  eb: the packed fields at the cell's left node; sf: the wave's
+// staged laser values (PGC).
 template <int M, bool STD, bool PGC>
-__device__ __forceinline__ void particle_terms(const JDepArgs &a, const double *sf, int c, int p, bool valid,
-                                               double x1, double x2, double pp1, double pp2, double pp3,
-                                               double qp, double psip, PartTerms<M> &t)
+__device__ __forceinline__ void particle_terms(const JDepArgs &a, uniform_ptr eb, const double *sf, int c, int p,
+                                               bool valid,
+                                               double x1, double x2, double pp1, double pp2, double pp3, double qp,
+                                               double psip, PartTerms<M> &t)
 {
     constexpr int NM = 2 * M + 1;
     double r = radius(x1, x2);
@@ -691,13 +762,12 @@ __device__ __forceinline__ void particle_terms(const JDepArgs &a, const double *
     double pos = __dmul_rn(r, a.idr);
     const double w1 = pos - (double)c, w0 = 1.0 - w1;
     double ep[3], bp[3];
-    gather3<M>(NodePairLds<NM>{sf}, w0, w1, pc, ps, ep);
-    gather3<M>(NodePairLds<NM>{sf + 6 * NM}, w0, w1, pc, ps, bp);
+    gather_eb<M>(eb, w0, w1, pc, ps, ep, bp, UniformFence());
     double gam_corr = 0.0;
     LaserAt la;
     if constexpr (PGC) {
-        la = gather_laser<M>(NodePairLds<NM, 1>{sf + 12 * NM}, NodePairLds<NM, 1>{sf + 14 * NM},
-                             NodePairLds<NM>{sf + 16 * NM}, NodePairLds<NM>{sf + 22 * NM}, w0, w1, pc, ps);
+        la = gather_laser<M>(NodePairLds<NM, 1>{sf}, NodePairLds<NM, 1>{sf + 2 * NM}, NodePairLds<NM>{sf + 4 * NM},
+                             NodePairLds<NM>{sf + 10 * NM}, w0, w1, pc, ps);
         gam_corr = 0.5 * a.qbm * a.qbm * (la.apr * la.apr + la.api * la.api);
     }
     // sqrt(1 + v^2) (+ gam_corr for the laser pushers)
@@ -866,18 +936,70 @@ __device__ __forceinline__ void mf_accumulate(double *rows, const PartTerms<M> &
     }
 }
 
-// Halving steps of the wave reduce-scatter applied to each pass's
-// contributions before they are accumulated: a lane keeps 16NM >> S
-// accumulators instead of 16NM, and the remaining 4 - S steps run once per
-// chunk.  Each step costs a chain of dependent cross-lane moves per pass, so
-// it pays only where the full set of accumulators would leave one wave per
-// SIMD: measured on MI355X (C2, M = 2: 20.6 us per launch with S = 0 and two
-// waves per SIMD, 23.1 us with S = 3 and four; C3, M = 4: 41.0 us with
-// S = 0 and one wave, 28.0 us with S = 1 and two).
+// The vector form of a wave's cell deposit: the same 16 x NM product as
+// outer-product tiles.  Each lane writes its particle's terms into the wave's
+// LDS rows ([val 0..7][ph 0..NM-1][w1], stride tile_stride); then lane
+// (g, q) = (lane / 4, lane % 4) reads the particles 16 j + g and adds the
+// 4 x NM products of tile q (both nodes, components 2q and 2q + 1) into its
+// own accumulators.  A lane so keeps 4 NM accumulators where a lane that
+// summed whole particles kept 16 NM, and the cross-lane sum at the end
+// exchanges 5 NM values instead of 17 NM.  Row groups past the pass's last
+// particle are skipped.
 template <int M>
-constexpr int dep_pass_steps()
+constexpr int tile_stride()
 {
-    return M <= 2 ? 0 : 1;
+    // even (16-byte reads) and = 2 mod 4 doubles, which spreads the rows over the LDS banks
+    return (10 + 2 * M) % 4 == 2 ? 10 + 2 * M : 12 + 2 * M;
+}
+
+template <int M>
+__device__ __forceinline__ void tile_accumulate(double *rows, const PartTerms<M> &t, int lane, int ngroups,
+                                                double (&acc)[4 * (2 * M + 1)])
+{
+    constexpr int NM = 2 * M + 1, STR = tile_stride<M>();
+    double2 *mine = reinterpret_cast<double2 *>(rows + lane * STR);
+#pragma unroll
+    for (int c = 0; c < 4; c++) mine[c] = make_double2(t.val[2 * c], t.val[2 * c + 1]);
+#pragma unroll
+    for (int k = 0; k <= M; k++) mine[4 + k] = make_double2(t.ph[2 * k], 2 * k + 1 < NM ? t.ph[2 * k + 1] : t.w[1]);
+    wave_lds_sync();
+    const int g = lane >> 2, q = lane & 3;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (j >= ngroups) break;
+        const double2 *r = reinterpret_cast<const double2 *>(rows + (16 * j + g) * STR);
+        const double2 v = r[q];
+        double ph[NM + 1];
+#pragma unroll
+        for (int k = 0; k <= M; k++) {
+            const double2 x = r[4 + k];
+            ph[2 * k] = x.x;
+            ph[2 * k + 1] = x.y;
+        }
+        const double w1 = ph[NM], w0 = 1.0 - w1;
+        const double av[4] = {w0 * v.x, w0 * v.y, w1 * v.x, w1 * v.y};
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int k = 0; k < NM; k++) acc[x * NM + k] += av[x] * ph[k];
+    }
+    wave_lds_sync();
+}
+
+// the 16 lane groups' tiles summed: row r of 16 lanes keeps the NM values of
+// node r / 2 and component 2 q + r % 2 (q = lane % 4), in acc[0 .. NM)
+template <int M>
+__device__ __forceinline__ void tile_reduce(double (&acc)[4 * (2 * M + 1)])
+{
+    constexpr int NM = 2 * M + 1;
+#pragma unroll
+    for (int i = 0; i < 2 * NM; i++) acc[i] = swap32_sum(acc[i], acc[2 * NM + i]);
+#pragma unroll
+    for (int i = 0; i < NM; i++) {
+        acc[i] = swap16_sum(acc[i], acc[NM + i]);
+        acc[i] = acc[i] + dpp<kDppRowRor8>(acc[i]);
+        acc[i] = acc[i] + dpp<kDppRowRor4>(acc[i]);
+    }
 }
 
 // the arguments of every species of one launch; workgroup row blockIdx.y
@@ -886,31 +1008,51 @@ struct JDepMulti {
     JDepArgs s[kMaxSpecies];
 };
 
+// waves per SIMD the compiler is asked to fit: the vector form of modes 0..2
+// lands a few VGPRs above the 128 that allow four
+template <int M, bool PGC, bool MF>
+constexpr int dep_min_waves() { return !MF && !PGC ? (M <= 2 ? 4 : 3) : 1; }
+
+// The current deposit's launch is bound by its longest wave and by the FP64
+// issue rate (420 FP64 instructions per 64 particles at modes 0..2), not by
+// its 48 B per particle.  MI355X, averages over the slices of a 3D step
+// through the driver and the first bubble (rocprofv3), first / later
+// iterations: 524,288 particles, 4096 cells, modes 0..2: 25.5 / 19.7 us with
+// 16 NM accumulators per lane, fields broadcast from LDS and one wave per
+// 1024-particle chunk, 20.0 / 14.6 us in this form; 2 x 131,072 particles,
+// 2048 cells, modes 0..4 (matrix form): 22.4 / 17.3 and 16.3 / 13.0 us.
+//
 // SPEC: a speculative launch of iteration >= 2 of a slice, which returns at
 // once when the iteration has already converged (a separate instance, so
 // that profiles show the first-iteration launches, which always work, apart)
 // MF: the matrix form of the accumulation (mf_accumulate) instead of the
-// reduce-scatter; the same values up to the order of the sums
+// vector form (tile_accumulate); the same values up to the order of the sums
 template <int M, bool SPEC, int CPW, bool STD, bool PGC = false, bool MF = false>
-__global__ __launch_bounds__(64 * CPW) void k_amjdeposit(const JDepMulti m)
+__global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF>())) void k_amjdeposit(const JDepMulti m)
 {
     const JDepArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     constexpr int NM = 2 * M + 1;
     constexpr int NV = 8 * NM;
     constexpr int NF = dep_staged<NM, PGC>();   // staged field values per cell
-    // the fields at the two nodes of each wave's cell (dep_staged layout)
+    constexpr int CH = crowd_chunks<CPW>(), PT = crowd_parts<CPW>();
+    // the laser fields at the two nodes of each wave's cell (PGC)
     __shared__ double sf[CPW][NF];
-    // the matrix form's particle rows, per wave
-    __shared__ double mrows[MF ? CPW * 32 * mf_stride<NM>() : 1];
+    // the particle rows of the wave's products, per wave
+    constexpr int ROWS = MF ? 32 * mf_stride<NM>() : 64 * tile_stride<M>();
+    __shared__ __align__(16) double mrows[CPW * ROWS];
+    // the part sums of crowded chunks
+    __shared__ double comb[CH][kDepSub][2 * NV];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (dep_group_idle<CPW>(a.nr, a.os)) return;
-    const DepChunk ch = dep_chunk<CPW>(a.nr, a.cs, a.os, a.desc, a.n_ov_max, wave);
-    const int c = ch.cell;
     const int nm = a.nm, ld = a.ld;
-    const int ix = c + 1;
+    const int ncg = (a.nr + CPW - 1) / CPW;
+    const bool crowd = (int)blockIdx.x >= ncg;
+    const int ncrowd = crowd ? min(a.os[a.nr + 1], a.n_crowd_max) : 0;
+    const int step = ((int)gridDim.x - ncg) * CH;
+    int o0 = ((int)blockIdx.x - ncg) * CH;
+    if (crowd && o0 >= ncrowd) return;
     // every independent load of the prologue first (one round trip): the
-    // convergence state, the cell's particle range and its field values
+    // convergence state and the cell's particle range (and laser values)
     int done = 0;
     double co = 0.0, cd = 0.0;
     int iters_now = 0;
@@ -919,20 +1061,27 @@ __global__ __launch_bounds__(64 * CPW) void k_amjdeposit(const JDepMulti m)
         iters_now = a.it->iters;
         conv_load(a.conv_prev, a.nblk, co, cd);
     }
-    const int p0 = ch.pb, p1 = ch.pe;
-    double fv[(NF + 63) / 64];
-#pragma unroll
-    for (int u = 0; u < (NF + 63) / 64; u++) {
-        const int l = min(lane + 64 * u, NF - 1);
-        if constexpr (PGC) {
-            fv[u] = dep_stage_load_pgc<NM>(a.e, a.b, a.ar, a.ai, a.arg, a.aig, nm, ld, l, ix);
-        } else {
-            const int fb = l / (6 * NM), r = l % (6 * NM);
-            const int n = r / (3 * NM), comp = (r / NM) % 3, k = r % NM;
-            const double *f = fb ? a.b : a.e;
-            fv[u] = f[((size_t)comp * nm + k) * ld + ix + n];
-        }
+    bool live = true;
+    DepRange rg;
+    int4 d = make_int4(0, 0, 0, 0);
+    const int ch = wave / (CPW / CH);
+    if (!crowd) {
+        rg = cell_range<CPW>(a.nr, a.cs, a.first, wave, live);
+    } else {
+        d = crowd_entry(a.desc, min(o0 + ch, ncrowd - 1));
+        rg.cell = d.x;
     }
+    uniform_ptr eb;
+    double fv[(NF + 63) / 64];
+    auto load_fields = [&](int c) {
+        eb = (uniform_ptr)(a.eb + (size_t)(c + 1) * (6 * NM));
+        if constexpr (PGC) {
+#pragma unroll
+            for (int u = 0; u < (NF + 63) / 64; u++)
+                fv[u] = dep_stage_load_pgc<NM>(a.ar, a.ai, a.arg, a.aig, nm, ld, min(lane + 64 * u, NF - 1), c + 1);
+        }
+    };
+    load_fields(rg.cell);
     if (SPEC) {
         int stop = done;
         if (!stop) {
@@ -950,77 +1099,109 @@ __global__ __launch_bounds__(64 * CPW) void k_amjdeposit(const JDepMulti m)
         }
         if (stop) return;
     }
-#pragma unroll
-    for (int u = 0; u < (NF + 63) / 64; u++) {
-        const int l = lane + 64 * u;
-        if (l < NF) sf[wave][l] = fv[u];
-    }
-    __syncthreads();
-    if (!ch.live) return;
+    if (!live) return;
     const double *__restrict__ X1 = a.x1;
     const double *__restrict__ X2 = a.x2;
     const double *__restrict__ PP1 = a.p1;
     const double *__restrict__ PP2 = a.p2;
     const double *__restrict__ PP3 = a.p3;
     const double *__restrict__ Q = a.q;
-    constexpr int S = dep_pass_steps<M>();
-    constexpr int NA = MF ? 1 : (2 * NV) >> S;
-    double acc[NA];
+    double acc[4 * NM];
+    dep_acc4 macc;
+    double *const wrows = mrows + wave * ROWS;
+    auto stage_fields = [&]() {
+        if constexpr (PGC) {
 #pragma unroll
-    for (int v = 0; v < NA; v++) acc[v] = 0.0;
-    dep_acc4 macc = {0.0, 0.0, 0.0, 0.0};
-    double *const wrows = mrows + (MF ? wave * 32 * mf_stride<NM>() : 0);
-    // every pass has all 64 lanes active (the exchanges need them); lanes
-    // past the chunk's end deposit zero.  Software-pipelined: the next pass's
-    // particle loads are in flight while this pass computes.
-    const int npass = __builtin_amdgcn_readfirstlane((p1 - p0 + 63) >> 6);
-    const int pl = max(p1 - 1, p0);
-    int p = p0 + lane;
-    int pc = min(p, pl);
-    double x1 = X1[pc], x2 = X2[pc], pp1 = PP1[pc], pp2 = PP2[pc], pp3 = PP3[pc], qp = Q[pc];
-    double psip = STD ? a.psi[pc] : 0.0;
-    for (int k = 0; k < npass; k++, p += 64) {
-        // the staged fields are re-read from LDS (broadcast) every particle
-        // rather than held in registers: the accumulators need the VGPRs
-        __asm__ volatile("" ::: "memory");
-        const int pn = min(p + 64, pl);
-        const double nx1 = X1[pn], nx2 = X2[pn], np1 = PP1[pn], np2 = PP2[pn], np3 = PP3[pn], nq = Q[pn];
-        const double npsi = STD ? a.psi[pn] : 0.0;
-        PartTerms<M> pt;
-        particle_terms<M, STD, PGC>(a, sf[wave], c, p, p < p1, x1, x2, pp1, pp2, pp3, qp, psip, pt);
+            for (int u = 0; u < (NF + 63) / 64; u++) {
+                const int l = lane + 64 * u;
+                if (l < NF) sf[wave][l] = fv[u];
+            }
+            wave_lds_sync();
+        }
+    };
+    // the wave's sums, value comp * NM + k of node ix to D0 and of node ix + 1 to D1
+    auto store = [&](double *D0, double *D1) {
         if constexpr (MF) {
-            mf_accumulate<M>(wrows, pt, lane, macc);
+            // lane l holds D[4 r + l / 16][l % 16]: row = node * 8 + comp, column = mode array
+            const int k = lane & 15, rb = lane >> 4;
+            if (k < NM) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int row = 4 * r + rb;
+                    (row < 8 ? D0 : D1)[(row & 7) * NM + k] = macc[r];
+                }
+            }
         } else {
-            const DepTerms<M> t(pt);
+            const int r = lane >> 4, comp = 2 * (lane & 3) + (r & 1), sub = (lane >> 2) & 3;
+            double *D = (r < 2 ? D0 : D1) + comp * NM;
 #pragma unroll
-            for (int i = 0; i < NA; i++) acc[i] += reduced_value<NM, S>(t, i, lane);
+            for (int k = 0; k < NM; k++)
+                if ((k & 3) == sub) D[k] = acc[k];
         }
-        x1 = nx1; x2 = nx2; pp1 = np1; pp2 = np2; pp3 = np3; qp = nq; psip = npsi;
-    }
-    double *D0 = ch.ovf ? a.O0 : a.P0, *D1 = ch.ovf ? a.O1 : a.P1;
-    if constexpr (MF) {
-        // lane l holds D[4 r + l / 16][l % 16]: row = node * 8 + comp, column = mode array
-        const int k = lane & 15, rb = lane >> 4;
-        const dep_acc4 sum = macc;
-        if (k < NM) {
+    };
+    stage_fields();
+    const int sub0 = (wave % (CPW / CH)) * PT;
+    int u = 0;
+    if (crowd) rg = part_range(d, sub0, o0 + ch < ncrowd);
+    for (;;) {
+        // the wave's sums over the particles of the range
+        const int c = rg.cell, p0 = rg.pb, p1 = rg.pe;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = 4 * r + rb, comp = row & 7;
-                double *D = row < 8 ? D0 : D1;
-                D[(size_t)ch.row * NV + comp * NM + k] = sum[r];
+        for (int v = 0; v < 4 * NM; v++) acc[v] = 0.0;
+        macc = dep_acc4{0.0, 0.0, 0.0, 0.0};
+        // every pass has all 64 lanes active (the exchanges need them); lanes
+        // past the range's end deposit zero.  Software-pipelined: the next
+        // pass's particle loads are in flight while this pass computes.
+        const int npass = __builtin_amdgcn_readfirstlane((p1 - p0 + 63) >> 6);
+        const int pl = max(p1 - 1, 0);
+        int p = p0 + lane;
+        int pc = min(p, pl);
+        double x1 = X1[pc], x2 = X2[pc], pp1 = PP1[pc], pp2 = PP2[pc], pp3 = PP3[pc], qp = Q[pc];
+        double psip = STD ? a.psi[pc] : 0.0;
+        for (int k = 0; k < npass; k++, p += 64) {
+            // the fields are read anew for every pass (scalar cache) rather
+            // than held in registers
+            UniformFence()(eb);
+            const int pn = min(p + 64, pl);
+            const double nx1 = X1[pn], nx2 = X2[pn], np1 = PP1[pn], np2 = PP2[pn], np3 = PP3[pn], nq = Q[pn];
+            const double npsi = STD ? a.psi[pn] : 0.0;
+            PartTerms<M> pt;
+            particle_terms<M, STD, PGC>(a, eb, sf[wave], c, p, p < p1, x1, x2, pp1, pp2, pp3, qp, psip, pt);
+            if constexpr (MF) {
+                mf_accumulate<M>(wrows, pt, lane, macc);
+            } else {
+                const int left = p1 - p0 - 64 * k;
+                tile_accumulate<M>(wrows, pt, lane, __builtin_amdgcn_readfirstlane((min(left, 64) + 15) >> 4), acc);
             }
+            x1 = nx1; x2 = nx2; pp1 = np1; pp2 = np2; pp3 = np3; qp = nq; psip = npsi;
         }
-    } else {
-        wave_reduce_from<NM, S>(acc);
-        const int g = lane >> 2;
-#pragma unroll
-        for (int i = 0; i < NM; i++) {
-            const int v = g * NM + i;
-            if ((lane & 3) == (i & 3)) {
-                if (v < NV) D0[(size_t)ch.row * NV + v] = acc[i];
-                else D1[(size_t)ch.row * NV + v - NV] = acc[i];
-            }
+        if constexpr (!MF) tile_reduce<M>(acc);
+        if (!crowd) {
+            store(a.P0 + (size_t)c * NV, a.P1 + (size_t)c * NV);
+            return;
         }
+        store(comb[ch][sub0 + u], comb[ch][sub0 + u] + NV);
+        if (++u < PT) {
+            rg = part_range(d, sub0 + u, o0 + ch < ncrowd);
+            continue;
+        }
+        u = 0;
+        __syncthreads();
+        for (int t = threadIdx.x; t < CH * 2 * NV; t += 64 * CPW) {
+            const int q = t / (2 * NV), v = t % (2 * NV);
+            if (o0 + q >= ncrowd) continue;
+            const int4 e = a.desc[o0 + q];
+            const double sum = ((comb[q][0][v] + comb[q][1][v]) + comb[q][2][v]) + comb[q][3][v];
+            double *D = e.w < 0 ? (v < NV ? a.P0 : a.P1) + (size_t)e.x * NV : (v < NV ? a.O0 : a.O1) + (size_t)e.w * NV;
+            D[v < NV ? v : v - NV] = sum;
+        }
+        o0 += step;
+        if (o0 >= ncrowd) return;
+        __syncthreads();
+        d = crowd_entry(a.desc, min(o0 + ch, ncrowd - 1));
+        load_fields(d.x);
+        stage_fields();
+        rg = part_range(d, sub0, o0 + ch < ncrowd);
     }
 }
 
@@ -1044,8 +1225,7 @@ static JDepArgs jdep_args(qpad_ctx *c, int s, int l, bool store_diag, bool repor
     a.psi = sp.psi;
     a.store_diag = store_diag;
     a.cs = sp.cell_start;
-    a.e = c->f[QPAD_F_E];
-    a.b = c->f[QPAD_F_B];
+    a.eb = c->eb;
     a.ar = c->f[QPAD_F_AR];
     a.ai = c->f[QPAD_F_AI];
     a.arg = c->f[QPAD_F_AR_GRAD];
@@ -1062,7 +1242,8 @@ static JDepArgs jdep_args(qpad_ctx *c, int s, int l, bool store_diag, bool repor
     a.desc = sp.ov_desc;
     a.O0 = sp.O0;
     a.O1 = sp.O1;
-    a.n_ov_max = sp.n_ov_max;
+    a.first = sp.dep_first;
+    a.n_crowd_max = sp.n_crowd_max;
     return a;
 }
 
@@ -1080,7 +1261,7 @@ static int launch_jdep_list(qpad_ctx *c, const int *list, int n, int l, bool sto
         const int s = list[i];
         // the report (the host's copy of the decision) from the first entry only
         m.s[i] = jdep_args(c, s, l, store_diag, report && i == 0);
-        gx = std::max(gx, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].n_ov_max, cpw));
+        gx = std::max(gx, dep_grid(c->g.nr, c->sp[s].npp, c->sp[s].dep_first, cpw));
     }
     dim3 grid((unsigned)gx, (unsigned)n), blk(64 * cpw);
     hipEvent_t stop = nullptr;
@@ -1178,7 +1359,7 @@ struct PushArgs {
     const double *psi;   // interpolated psi (standard pusher)
     const int32_t *cs;
     uint32_t *key;
-    const double *e, *b;
+    const double *eb;   // the packed E and B of the slice
     const double *ar, *ai, *arg, *aig;   // laser envelope and gradients (PGC)
 };
 
@@ -1212,8 +1393,7 @@ __global__ __launch_bounds__(256) void k_push(const PushMulti m)
     const int ix = ic + 1;
     const double w1 = pos - (double)ic, w0 = 1.0 - w1;
     double ep[3], bp[3];
-    gather3<M>(NodePair{a.e, nm, ld, ix}, w0, w1, pc, ps, ep);
-    gather3<M>(NodePair{a.b, nm, ld, ix}, w0, w1, pc, ps, bp);
+    gather_eb<M>(a.eb + (size_t)ix * (6 * (2 * M + 1)), w0, w1, pc, ps, ep, bp, NoFence());
     double t = ep[0] * pc - ep[1] * ps;
     ep[1] = ep[0] * ps + ep[1] * pc;
     ep[0] = t;
@@ -1323,8 +1503,7 @@ static PushArgs push_args(qpad_ctx *c, int s)
     a.psi = sp.psi;
     a.cs = sp.cell_start;
     a.key = sp.key;
-    a.e = c->f[QPAD_F_E];
-    a.b = c->f[QPAD_F_B];
+    a.eb = c->eb;
     a.ar = c->f[QPAD_F_AR];
     a.ai = c->f[QPAD_F_AI];
     a.arg = c->f[QPAD_F_AR_GRAD];

@@ -390,6 +390,7 @@ struct BfieldArgs {
     FieldCommon g;
     const double *src, *b_beam, *psi;
     double *b_spe, *b_out, *e;
+    double *eb;         // e and b packed per node (qpad_ctx::eb)
     double *conv_re, *conv_im;
     double *conv_blk;   // this iteration's half: [workgroup][max old^2, max diff^2]
     IterState *it;
@@ -397,21 +398,24 @@ struct BfieldArgs {
     int late_done;      // as in SrcArgs
 };
 
-// thread per node i = 0..nr+1, all modes: B_r, B_phi of b_spe from the
-// B+/B- solutions (field_b_class.f03:715-752), b = b_spe + b_beam, E_perp
-// (field_e_class.f03:443-504), and convergence_tester 'compare'
-// (simulation_class.f03:560-599): the node's sum_m |B_phi,m| against the
-// recorded one, max over the workgroup's nodes (the next iteration's deposit
-// reduces the workgroup maxima).  Loads are issued for all modes before any
-// arithmetic.
+// workgroup of kBfThreads nodes i = 0..nr+1, a wave per mode m: B_r, B_phi of
+// b_spe from the B+/B- solutions (field_b_class.f03:715-752), b = b_spe +
+// b_beam, E_perp (field_e_class.f03:443-504), the packed fields, and
+// convergence_tester 'compare' (simulation_class.f03:560-599): the node's
+// sum_m |B_phi,m| against the recorded one (the modes' values meet in LDS and
+// are added in mode order), max over the workgroup's nodes (the next
+// iteration's deposit reduces the workgroup maxima).  Latency-bound: a wave
+// per mode keeps each thread's loads (all issued before any arithmetic) and
+// stores few.
 static_assert((16 * kSolveThreads + 2 + kBfThreads - 1) / kBfThreads <= kConvMaxBlocks,
               "the next deposit reduces every B_perp workgroup's maxima");
+static_assert(kBfThreads == 64, "a wave per mode");
 
 template <int M>
-__global__ __launch_bounds__(kBfThreads) void k_bfields(BfieldArgs a)
+__global__ __launch_bounds__(kBfThreads *(M + 1)) void k_bfields(BfieldArgs a)
 {
     constexpr int NM = 2 * M + 1;
-    __shared__ double red[8];
+    __shared__ double vabs[M + 1][2][kBfThreads];   // |Re B_phi,m|, |Im B_phi,m|
     // tested once the loads are requested (late_done); a vector load
     int done = flag_vload(&a.it->done);
     if (!a.late_done) {
@@ -420,88 +424,111 @@ __global__ __launch_bounds__(kBfThreads) void k_bfields(BfieldArgs a)
     }
     const FieldCommon &g = a.g;
     const int nm = NM, ld = g.ld, nr = g.nr;
-    const int t = threadIdx.x;
-    const int i = blockIdx.x * blockDim.x + t;
+    const int t = threadIdx.x & 63;
+    const int m = M == 0 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = blockIdx.x * kBfThreads + t;
     const bool valid = i <= nr + 1;
     const int ic = min(i, nr + 1);
     const bool inner = valid && ic >= 1 && ic <= nr;
     const int r = min(max(ic - 1, 0), nr - 1);
+    const int k0 = m == 0 ? 0 : 2 * m - 1;          // the mode's arrays: k0 and (m > 0) k0 + 1
     // ---- loads ----
-    double raw[M + 1][4], bb[NM][3], bs[NM][3], pw[NM][4], pp_i[NM], pp_2[NM];
+    double raw[4], bb[2][3], bz[2], pw[2][4], pp_i[2], pp_2[2], ez[2];
 #pragma unroll
-    for (int m = 0; m <= M; m++)
+    for (int q = 0; q < 4; q++) raw[q] = a.src[(size_t)(4 * m + q) * nr + r];
 #pragma unroll
-        for (int q = 0; q < 4; q++) raw[m][q] = a.src[(size_t)(4 * m + q) * nr + r];
-#pragma unroll
-    for (int k = 0; k < NM; k++) {
+    for (int u = 0; u < 2; u++) {
+        const int k = m == 0 ? 0 : k0 + u;
         const int p = k == 0 ? 0 : ((k & 1) ? k + 1 : k - 1);
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            bb[k][c] = FX(a.b_beam, c, k, ic);
-            bs[k][c] = FX(a.b_spe, c, k, ic);
-        }
+        for (int c = 0; c < 3; c++) bb[u][c] = FX(a.b_beam, c, k, ic);
+        bz[u] = FX(a.b_spe, 2, k, ic);
+        ez[u] = FX(a.e, 2, k, ic);
 #pragma unroll
-        for (int w = 0; w < 4; w++) pw[k][w] = a.psi[(size_t)k * ld + min(max(ic - 2 + w, 0), nr + 1)];
-        pp_i[k] = a.psi[(size_t)p * ld + ic];
-        pp_2[k] = a.psi[(size_t)p * ld + 2];
+        for (int w = 0; w < 4; w++) pw[u][w] = a.psi[(size_t)k * ld + min(max(ic - 2 + w, 0), nr + 1)];
+        pp_i[u] = a.psi[(size_t)p * ld + ic];
+        pp_2[u] = a.psi[(size_t)p * ld + 2];
     }
-    const double ore = a.conv_re[ic], oim = a.conv_im[ic];
+    double ore = 0.0, oim = 0.0;
+    if (m == 0) {
+        ore = a.conv_re[ic];
+        oim = a.conv_im[ic];
+    }
     if (a.late_done) {
         __asm__ volatile("" : "+v"(done));
         if (__builtin_amdgcn_readfirstlane(done)) return;
     }
     // ---- b_spe (inner nodes), b, E_perp ----
-#pragma unroll
-    for (int m = 0; m <= M; m++) {
-        if (!inner) break;
-        const int kr = m == 0 ? 0 : 2 * m - 1, ki = 2 * m;
-        const double sv[4] = {raw[m][0], m ? raw[m][1] : 0.0, raw[m][2], m ? raw[m][3] : 0.0};
+    double bs[2][2];
+    if (inner) {
+        const double sv[4] = {raw[0], m ? raw[1] : 0.0, raw[2], m ? raw[3] : 0.0};
         double o[4];
         bpm_recombine(m, ic, sv, o);
-        bs[kr][0] = o[0];
-        bs[kr][1] = o[2];
-        if (m > 0) {
-            bs[ki][0] = o[1];
-            bs[ki][1] = o[3];
-        }
-    }
-    double sre = 0.0, sim = 0.0, dre = ore, dim = oim;
-#pragma unroll
-    for (int m = 0; m <= M; m++) {
-        const double vr = fabs(bs[m == 0 ? 0 : 2 * m - 1][1]);
-        dre = dre - vr;
-        sre = sre + vr;
-        if (m > 0) {
-            const double vi = fabs(bs[2 * m][1]);
-            dim = dim - vi;
-            sim = sim + vi;
-        }
+        bs[0][0] = o[0];
+        bs[0][1] = o[2];
+        bs[1][0] = o[1];
+        bs[1][1] = o[3];
+        vabs[m][0][t] = fabs(bs[0][1]);
+        vabs[m][1][t] = fabs(bs[1][1]);
     }
     if (valid) {
 #pragma unroll
-        for (int k = 0; k < NM; k++) {
-            const double br = bs[k][0] + bb[k][0], bphi = bs[k][1] + bb[k][1];
+        for (int u = 0; u < 2; u++) {
+            if (u == 1 && m == 0) break;
+            const int k = k0 + u;
+            if (!inner) {
+                bs[u][0] = FX(a.b_spe, 0, k, ic);
+                bs[u][1] = FX(a.b_spe, 1, k, ic);
+            }
+            const double br = bs[u][0] + bb[u][0], bphi = bs[u][1] + bb[u][1], bzt = bz[u] + bb[u][2];
+            double ev[2];
+            if (inner) {
+                et_window(g, br, bphi, pw[u][0], pw[u][1], pw[u][2], pw[u][3], pp_i[u], pp_2[u], k, ic, ev);
+            } else {
+                ev[0] = FX(a.e, 0, k, ic);
+                ev[1] = FX(a.e, 1, k, ic);
+            }
+            double2 *eb = reinterpret_cast<double2 *>(a.eb + ((size_t)ic * NM + k) * 6);
+            eb[0] = make_double2(ev[0], ev[1]);
+            eb[1] = make_double2(ez[u], br);
+            eb[2] = make_double2(bphi, bzt);
             FX(a.b_out, 0, k, ic) = br;
             FX(a.b_out, 1, k, ic) = bphi;
-            FX(a.b_out, 2, k, ic) = bs[k][2] + bb[k][2];
-            if (!inner) continue;
-            FX(a.b_spe, 0, k, ic) = bs[k][0];
-            FX(a.b_spe, 1, k, ic) = bs[k][1];
-            double ev[2];
-            et_window(g, br, bphi, pw[k][0], pw[k][1], pw[k][2], pw[k][3], pp_i[k], pp_2[k], k, ic, ev);
-            FX(a.e, 0, k, ic) = ev[0];
-            FX(a.e, 1, k, ic) = ev[1];
+            FX(a.b_out, 2, k, ic) = bzt;
+            if (inner) {
+                FX(a.b_spe, 0, k, ic) = bs[u][0];
+                FX(a.b_spe, 1, k, ic) = bs[u][1];
+                FX(a.e, 0, k, ic) = ev[0];
+                FX(a.e, 1, k, ic) = ev[1];
+            }
         }
     }
+    if (M > 0) __syncthreads();
+    if (m > 0) return;
     double mx_old = -INFINITY, mx_d = -INFINITY;
     if (inner) {
+        double sre = 0.0, sim = 0.0, dre = ore, dim = oim;
+#pragma unroll
+        for (int q = 0; q <= M; q++) {
+            const double vr = vabs[q][0][t];
+            dre = dre - vr;
+            sre = sre + vr;
+            if (q > 0) {
+                const double vi = vabs[q][1][t];
+                dim = dim - vi;
+                sim = sim + vi;
+            }
+        }
         mx_old = ore * ore + oim * oim;
         mx_d = dre * dre + dim * dim;
         a.conv_re[ic] = sre;
         a.conv_im[ic] = sim;
     }
-    mx_old = block_max(mx_old, red);
-    mx_d = block_max(mx_d, red);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        mx_old = fmax(mx_old, __shfl_xor(mx_old, d, 64));
+        mx_d = fmax(mx_d, __shfl_xor(mx_d, d, 64));
+    }
     if (t == 0) {
         a.conv_blk[2 * blockIdx.x] = mx_old;
         a.conv_blk[2 * blockIdx.x + 1] = mx_d;
@@ -561,13 +588,14 @@ int launch_iteration_fields(qpad_ctx *c, int j, int l)
     f.b_spe = c->f[QPAD_F_B_SPE];
     f.b_out = c->f[QPAD_F_B];
     f.e = c->f[QPAD_F_E];
+    f.eb = c->eb;
     f.conv_re = c->conv_re;
     f.conv_im = c->conv_im;
     f.conv_blk = c->conv_blk + (size_t)(l & 1) * 2 * conv_blocks(c->g.nr);
     f.it = c->it;
     f.l = l;
     f.late_done = c->adaptive;
-    const dim3 fgrid((unsigned)conv_blocks(c->g.nr)), fblk(kBfThreads);
+    const dim3 fgrid((unsigned)conv_blocks(c->g.nr)), fblk(kBfThreads * (c->g.M + 1));
     switch (c->g.M) {
     case 0: hipLaunchKernelGGL(k_bfields<0>, fgrid, fblk, 0, c->stream, f); break;
     case 1: hipLaunchKernelGGL(k_bfields<1>, fgrid, fblk, 0, c->stream, f); break;
@@ -836,6 +864,7 @@ struct EperpArgs {
     double *b_spe;
     const double *b_beam, *psi;
     double *b_out, *e;
+    double *eb;         // e and b packed per node (qpad_ctx::eb)
     // learned seed of the iteration (B_perp components 0, 1 of nodes
     // 1..nr), copied into b_spe here, or null
     const double *seed;
@@ -882,11 +911,41 @@ __global__ __launch_bounds__(kNodeThreads) void k_eperp(EperpArgs a)
         bv[c] = bs + FX(a.b_beam, c, k, i);
         FX(a.b_out, c, k, i) = bv[c];
     }
-    if (!inner) return;
     double ev[2];
-    et_node(g, bv[0], bv[1], FieldArr{a.psi, nm, ld}, k, i, ev);
-    FX(a.e, 0, k, i) = ev[0];
-    FX(a.e, 1, k, i) = ev[1];
+    if (inner) {
+        et_node(g, bv[0], bv[1], FieldArr{a.psi, nm, ld}, k, i, ev);
+        FX(a.e, 0, k, i) = ev[0];
+        FX(a.e, 1, k, i) = ev[1];
+    } else {
+        ev[0] = FX(a.e, 0, k, i);
+        ev[1] = FX(a.e, 1, k, i);
+    }
+    double2 *eb = reinterpret_cast<double2 *>(a.eb + ((size_t)i * nm + k) * 6);
+    eb[0] = make_double2(ev[0], ev[1]);
+    eb[1] = make_double2(FX(a.e, 2, k, i), bv[0]);
+    eb[2] = make_double2(bv[1], bv[2]);
+}
+
+// thread per (node i = 0..nr+1, mode array k): e and b into the packed
+// fields (the fine-grained calls, whose e and b come from separate solves)
+__global__ __launch_bounds__(kNodeThreads) void k_pack_eb(const double *e, const double *b, double *eb, int nr, int nm,
+                                                          int ld)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = blockIdx.y;
+    if (i > nr + 1) return;
+    double2 *o = reinterpret_cast<double2 *>(eb + ((size_t)i * nm + k) * 6);
+    o[0] = make_double2(FX(e, 0, k, i), FX(e, 1, k, i));
+    o[1] = make_double2(FX(e, 2, k, i), FX(b, 0, k, i));
+    o[2] = make_double2(FX(b, 1, k, i), FX(b, 2, k, i));
+}
+
+int launch_pack_eb(qpad_ctx *c)
+{
+    hipLaunchKernelGGL(k_pack_eb, dim3((unsigned)node_blocks(c->g.nr), c->g.nm), dim3(kNodeThreads), 0, c->stream,
+                       c->f[QPAD_F_E], c->f[QPAD_F_B], c->eb, c->g.nr, c->g.nm, c->g.ld);
+    QPAD_HIP_CHECK(hipGetLastError());
+    return 0;
 }
 
 int src_rows_host(int M, int nm) { return src_rows(M, nm); }
@@ -952,6 +1011,7 @@ int launch_start_eperp(qpad_ctx *c, int j, const double *seed)
     e.psi = c->f[QPAD_F_PSI];
     e.b_out = c->f[QPAD_F_B];
     e.e = c->f[QPAD_F_E];
+    e.eb = c->eb;
     e.seed = seed;
     e.conv_re = c->conv_re;
     e.conv_im = c->conv_im;

@@ -13,8 +13,9 @@
 //                   particles with the same key, in the fixed order (round,
 //                   wave, lane), from wave ballots; position = cell_start +
 //                   chunk offset + rank; moves every particle array.
-//                   Workgroup 0 also lists the deposit's overflow chunks
-//                   (cells holding more than kDepChunk particles).
+//                   Workgroup 0 also numbers the overflow rows of cells
+//                   holding more than kDepChunk particles and lists the
+//                   crowded cells' chunks for the deposits.
 // Integer counting only, in a fixed order: the permutation is the same on
 // every run.
 #include <algorithm>
@@ -45,9 +46,9 @@ struct SortArgs {
     double *d[8];
     const int32_t *sid;
     int32_t *did;
-    int32_t *os;            // [nb] overflow rows of cell c: os[c] .. os[c+1]-1
-    int4 *desc;             // [n_ov_max] (cell, first particle, end, 0)
-    int n_ov_max;
+    int32_t *os;            // [nb] overflow rows of cell c: os[c] .. os[c+1]-1; [nb] crowded chunks
+    int4 *desc;             // [n_crowd_max] (cell, first particle, end, overflow row or -1)
+    int n_ov_max, n_crowd_max, first;
 };
 
 // the arguments of every species of one launch (workgroup rows by species)
@@ -174,49 +175,56 @@ __device__ inline void scan_totals(const SortArgs &a, int *base)
 }
 
 // workgroup 0, after scan_totals: cell c < nr (nr = nb - 1) with n_c
-// particles is deposited in chunks of kDepChunk; chunk 0 by the cell's own
-// wave, chunks 1 .. ceil(n_c / kDepChunk) - 1 by overflow waves.  Their rows
-// are numbered cell by cell, chunk by chunk: os = exclusive prefix of the
-// chunk counts, desc[row] = (cell, first particle, end)
+// particles is deposited in chunks of kDepChunk: chunk 0 into the cell's own
+// partial row, chunks 1 .. into overflow rows, numbered cell by cell, chunk
+// by chunk (os = exclusive prefix of their counts).  The chunks of cells of
+// more than `first` particles are the crowded list of the deposits: desc =
+// (cell, first particle, end, overflow row; -1: the cell's own row), their
+// number at os[nr + 1].
 __device__ inline void overflow_chunks(const SortArgs &a, const int *base)
 {
-    __shared__ int wsum[kSortThreads / 64];
+    __shared__ uint64_t wsum[kSortThreads / 64];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int nr = a.nb - 1;
     const int per = (nr + kSortThreads - 1) / kSortThreads;
     const int c0 = t * per;
-    int local = 0;
-    for (int q = 0; q < per; q++) {
-        const int c = c0 + q;
-        if (c < nr) {
-            const int n = base[c + 1] - base[c];
-            local += n > 0 ? (n - 1) / kDepChunk : 0;
-        }
-    }
-    int incl = local;
+    // overflow rows (low half) and crowded chunks (high half) of n particles
+    auto rows_of = [&](int n) -> uint64_t {
+        const uint64_t k = n > 0 ? (uint64_t)((n - 1) / kDepChunk) : 0;
+        return k | (n > a.first ? (k + 1) << 32 : 0);
+    };
+    uint64_t local = 0;
+    for (int q = 0; q < per; q++)
+        if (c0 + q < nr) local += rows_of(base[c0 + q + 1] - base[c0 + q]);
+    uint64_t incl = local;
     for (int dd = 1; dd < 64; dd <<= 1) {
-        const int y = __shfl_up(incl, dd, 64);
+        const uint64_t y = __shfl_up(incl, dd, 64);
         if (lane >= dd) incl += y;
     }
     if (lane == 63) wsum[wave] = incl;
     __syncthreads();
-    int run = incl - local;
+    uint64_t run = incl - local;
     for (int w = 0; w < wave; w++) run += wsum[w];
     for (int q = 0; q < per; q++) {
         const int c = c0 + q;
         if (c >= nr) break;
         const int p0 = base[c], p1 = base[c + 1];
-        const int k = p1 > p0 ? (p1 - p0 - 1) / kDepChunk : 0;
-        a.os[c] = min(run, a.n_ov_max);
-        for (int u = 1; u <= k; u++) {
-            const int row = run + u - 1;
-            if (row < a.n_ov_max) a.desc[row] = make_int4(c, p0 + u * kDepChunk, min(p0 + (u + 1) * kDepChunk, p1), 0);
-        }
+        const uint64_t k = rows_of(p1 - p0);
+        const int row0 = (int)(uint32_t)run, at = (int)(run >> 32), chunks = (int)(k >> 32);
+        a.os[c] = min(row0, a.n_ov_max);
+        for (int u = 0; u < chunks; u++)
+            if (at + u < a.n_crowd_max)
+                a.desc[at + u] = make_int4(c, p0 + u * kDepChunk, min(p0 + (u + 1) * kDepChunk, p1),
+                                           u == 0 ? -1 : min(row0 + u - 1, a.n_ov_max - 1));
         run += k;
     }
-    // the last thread's running count is the total (its range may be empty);
-    // rows never exceed n_ov_max (the chunks of n particles number < n / kDepChunk)
-    if (t == kSortThreads - 1) a.os[nr] = min(run, a.n_ov_max);
+    // the last thread's running counts are the totals (its range may be
+    // empty); overflow rows never exceed n_ov_max (the chunks of n particles
+    // number < n / kDepChunk), crowded chunks never n_crowd_max
+    if (t == kSortThreads - 1) {
+        a.os[nr] = min((int)(uint32_t)run, a.n_ov_max);
+        a.os[nr + 1] = min((int)(run >> 32), a.n_crowd_max);
+    }
 }
 
 __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const SortMulti m)
@@ -354,6 +362,8 @@ static SortArgs sort_args(qpad_ctx *c, int s)
     a.os = sp.ov_start;
     a.desc = sp.ov_desc;
     a.n_ov_max = sp.n_ov_max;
+    a.n_crowd_max = sp.n_crowd_max;
+    a.first = sp.dep_first;
     return a;
 }
 

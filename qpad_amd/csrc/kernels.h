@@ -38,6 +38,8 @@ int launch_compare_only(qpad_ctx *c);
 // (k_solve), then b_spe, b, E_perp and the convergence maxima (k_bfields);
 // each returns at once once the iteration has converged
 int launch_iteration_fields(qpad_ctx *c, int j, int l);
+// the packed fields (qpad_ctx::eb) from the e and b slice fields
+int launch_pack_eb(qpad_ctx *c);
 // slice epilogue: cbq, e_spe, history copies, beam fields of slice j, the
 // J_perp predictor for the next slice
 int launch_epilogue(qpad_ctx *c, int j);

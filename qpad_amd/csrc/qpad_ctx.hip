@@ -421,6 +421,7 @@ int qpad_create(const qpad_grid *gr, qpad_ctx **out)
         c->ncomp[f] = ncomp[f];
         rc = dalloc(&c->f[f], f1_size(c, ncomp[f]));
     }
+    if (!rc) rc = dalloc(&c->eb, ((size_t)g.nr + 2) * 6 * g.nm);
     const size_t ns = (size_t)g.nxi + 2;
     if (!rc) rc = dalloc(&c->h_psi, ns * f1_size(c, 1));
     if (!rc) rc = dalloc(&c->h_e, ns * f1_size(c, 3));
@@ -496,6 +497,7 @@ int qpad_create(const qpad_grid *gr, qpad_ctx **out)
     if (he != hipSuccess) rc = fail(QPAD_E_HIP, "upload of solver factors failed");
     // zero every array once (fill kernels, not memset)
     for (int f = 0; f < QPAD_NFIELD && !rc; f++) rc = zero_dev(c, c->f[f], f1_size(c, c->ncomp[f]));
+    if (!rc) rc = zero_dev(c, c->eb, ((size_t)g.nr + 2) * 6 * g.nm);
     double *hs[] = {c->h_psi, c->h_q_spe, c->h_q_beam};
     for (double *h : hs)
         if (!rc) rc = zero_dev(c, h, ns * f1_size(c, 1));
@@ -527,7 +529,7 @@ int qpad_destroy(qpad_ctx *c)
     dfree(c->h_psi); dfree(c->h_e); dfree(c->h_b); dfree(c->h_b_spe); dfree(c->h_e_spe);
     dfree(c->h_cu); dfree(c->h_q_spe); dfree(c->h_q_beam); dfree(c->h_b_beam);
     dfree(c->conv_re); dfree(c->conv_im); dfree(c->conv_blk); dfree(c->it); dfree(c->fac); dfree(c->src);
-    dfree(c->sc_ef);
+    dfree(c->sc_ef); dfree(c->eb);
     if (c->sc_ef_host) (void)hipHostFree(c->sc_ef_host);
     dfree(c->lz_ar); dfree(c->lz_ai); dfree(c->h_chi);
     if (c->it_host) (void)hipHostFree(c->it_host);
@@ -600,12 +602,17 @@ static int species_create(qpad_ctx *c, const qpad_species_cfg *cfg, const qpad_n
     if (!rc) rc = dalloc(&sp.P0, (size_t)c->g.nr * 8 * c->g.nm);
     if (!rc) rc = dalloc(&sp.P1, (size_t)c->g.nr * 8 * c->g.nm);
     sp.n_ov_max = (int)(sp.npmax / kDepChunk + 1);
-    if (!rc) rc = dalloc(&sp.ov_start, (size_t)c->g.nr + 1);
-    if (!rc) rc = dalloc(&sp.ov_desc, (size_t)sp.n_ov_max);
+    // a wave takes cells of up to twice the injected particles per cell (at
+    // least four passes, at most one chunk)
+    const int64_t per_cell = (int64_t)cfg->ppc1 * cfg->ppc2 * cfg->num_theta;
+    sp.dep_first = (int)std::min<int64_t>(std::max<int64_t>((2 * per_cell + 63) / 64 * 64, kDepFirstMin), kDepChunk);
+    sp.n_crowd_max = (int)(sp.npmax / (sp.dep_first + 1) + sp.npmax / kDepChunk + 1);
+    if (!rc) rc = dalloc(&sp.ov_start, (size_t)c->g.nr + 2);
+    if (!rc) rc = dalloc(&sp.ov_desc, (size_t)sp.n_crowd_max);
     if (!rc) rc = dalloc(&sp.O0, (size_t)sp.n_ov_max * 8 * c->g.nm);
     if (!rc) rc = dalloc(&sp.O1, (size_t)sp.n_ov_max * 8 * c->g.nm);
-    if (!rc && (hipMemsetAsync(sp.ov_start, 0, sizeof(int32_t) * ((size_t)c->g.nr + 1), c->stream) != hipSuccess ||
-                hipMemsetAsync(sp.ov_desc, 0, sizeof(int4) * (size_t)sp.n_ov_max, c->stream) != hipSuccess))
+    if (!rc && (hipMemsetAsync(sp.ov_start, 0, sizeof(int32_t) * ((size_t)c->g.nr + 2), c->stream) != hipSuccess ||
+                hipMemsetAsync(sp.ov_desc, 0, sizeof(int4) * (size_t)sp.n_crowd_max, c->stream) != hipSuccess))
         rc = fail(QPAD_E_HIP, "hipMemsetAsync of the overflow rows failed");
     if (!rc) rc = dalloc(&sp.hist, hist_ints);
     if (!rc) rc = dalloc(&sp.tot, (size_t)c->g.nr + 1);
@@ -1298,6 +1305,7 @@ int qpad_species_amjdp(qpad_ctx *c, int32_t s, double dxi)
 {
     if (!c || s < 0 || s >= c->nspecies) return fail(QPAD_E_INVALID, "bad species");
     if (!(dxi > 0.0 && dxi < INFINITY)) return fail(QPAD_E_INVALID, "dxi must be > 0");
+    TRY(launch_pack_eb(c));
     c->dt2d = dxi;
     const int rc = launch_amjdeposit(c, s, 0, true, false);
     c->dt2d = c->g.dxi;
@@ -1390,6 +1398,7 @@ static int species_push(qpad_ctx *c, int32_t s, double dxi, double clamp)
 {
     if (!c || s < 0 || s >= c->nspecies) return fail(QPAD_E_INVALID, "bad species");
     if (!(dxi > 0.0 && dxi < INFINITY)) return fail(QPAD_E_INVALID, "dxi must be > 0");
+    TRY(launch_pack_eb(c));
     c->dt2d = dxi;
     c->clamp2d = clamp;
     int rc = launch_push(c, s);

@@ -22,11 +22,13 @@ constexpr int kMaxSpecies = 4;
 constexpr int kMaxBeams = 4;
 constexpr int kSolveThreads = 512;   // workgroup of the tridiagonal solves
 constexpr int kDepWaves = 4;         // default radial cells (waves) per deposit workgroup
-// particles per deposit wave: a cell holding more is deposited in chunks of
-// kDepChunk, the first by the cell's own wave, the others by overflow waves
-// with partials of their own (rows of Species::O0/O1), so that a crowded
-// cell no longer holds up a whole deposit launch
+// a cell holding more particles is deposited in chunks of kDepChunk, the
+// first into the cell's own partial row, the others into rows of their own
+// (Species::O0/O1), so that a crowded cell does not hold up a whole deposit
+// launch; a chunk is shared by the four waves of a workgroup where its cell
+// holds more than Species::dep_first particles
 constexpr int kDepChunk = 1024;
+constexpr int kDepFirstMin = 256;
 
 // field kinds (source/param.f03:75-84)
 enum { FK_PSI = 0, FK_EZ = 1, FK_BZ = 2, FK_BT = 3, FK_BPLUS = 4, FK_BMINUS = 5, FK_N = 6 };
@@ -55,13 +57,16 @@ struct Species {
     int32_t *cell_start;     // nr + 2 entries, cell_start[nr] = live count
     double *qn;              // neutralising background, 1 x nm x ld
     double *P0, *P1;         // per-cell deposit partials [nr][nval] (first chunk)
-    // overflow chunks of crowded cells (written by the sort): rows
-    // ov_start[c] .. ov_start[c+1]-1 belong to cell c, in particle order;
-    // ov_desc[row] = (cell, first particle, end, 0); O0/O1 [row][nval]
-    int32_t *ov_start;       // nr + 1 entries, ov_start[nr] = rows in use
+    // crowded cells (written by the sort): overflow rows ov_start[c] ..
+    // ov_start[c+1]-1 belong to cell c, in particle order, O0/O1 [row][nval];
+    // ov_desc = the chunks (cell, first particle, end, overflow row or -1
+    // for the cell's own row) of the cells of more than dep_first particles
+    int32_t *ov_start;       // nr + 2 entries, [nr] = overflow rows, [nr + 1] = chunks listed
     int4 *ov_desc;
     double *O0, *O1;
     int n_ov_max;            // rows allocated: npmax / kDepChunk + 1
+    int dep_first;           // most particles of a cell that one wave deposits
+    int n_crowd_max;         // chunks ov_desc holds
     int *hist, *tot;         // counting-sort workspace: [chunks][nr+1], [nr+1]
     // species2d%q and its history (cbq), kept when the context tracks the
     // per-species charge (qpad_species_charge_history): 1 x nm x ld and
@@ -141,6 +146,10 @@ struct qpad_ctx {
     // slice fields
     double *f[QPAD_NFIELD];
     int ncomp[QPAD_NFIELD];
+    // E and B of the slice packed for the gathers of the current deposit and
+    // the push: [node 0..nr+1][k][e_r, e_phi, e_z, b_r, b_phi, b_z]; written
+    // with e and b by the slice's field kernels (launch_pack_eb elsewhere)
+    double *eb;
     // histories (slices 0..nxi+1)
     double *h_psi, *h_e, *h_b, *h_b_spe, *h_e_spe, *h_cu, *h_q_spe, *h_q_beam, *h_b_beam;
     // solver factors [kind][mode][lo|inv|cp][K * kSolveThreads], transposed

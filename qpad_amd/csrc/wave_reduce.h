@@ -68,6 +68,8 @@ constexpr int kDppRowMirror = 0x140;
 constexpr int kDppRowHalfMirror = 0x141;
 constexpr int kDppQuadXor1 = 0xB1;   // quad_perm [1, 0, 3, 2]
 constexpr int kDppQuadXor2 = 0x4E;   // quad_perm [2, 3, 0, 1]
+constexpr int kDppRowRor4 = 0x124;   // rotations within 16 lanes
+constexpr int kDppRowRor8 = 0x128;
 
 // One exchange step of the reduce-scatter.  Level L (0..4) holds
 // 16 NB >> L values per lane; step L -> L + 1 pairs value i with value
