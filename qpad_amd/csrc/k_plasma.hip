@@ -16,6 +16,7 @@
 
 #include "kernels.h"
 #include "sort_config.h"
+#include "sort_device.h"
 #include "rng.h"
 #include "wave_reduce.h"
 #include "conv.h"
@@ -1346,21 +1347,28 @@ int launch_amjdeposit_all(qpad_ctx *c, int l, bool store_diag, bool timed, bool 
 }
 
 // ---------------------------------------------------------------------------
-// push_u_robust (part2d_class.f03:1879-1965) + push_x (:2221-2262) + the new
-// sort key (update_bound :2307-2353 is the key nr).  Thread per particle;
-// particles that already left the box (past cell_start[nr]) keep key nr.
+// push_u_robust (part2d_class.f03:1879-1965) + push_x (:2221-2262) + the
+// re-sort by the new cells (update_bound :2307-2353 is the key nr).
+// Particles that already left the box (past cell_start[nr]) keep key nr.
+// Two forms, by the number of particles (SortArgs::direct):
+// - few particles: two launches.  The counting pass pushes them only for
+//   their new cells, the scattering pass pushes them again on the way to their
+//   sorted places; the launches' latencies are all that counts (blowout
+//   deck, 4096 particles in 256 cells, MI355X: push + counting + scan +
+//   scatter 5.4 + 2.9 + 2.8 + 13.0 us, now 5.0 + 6.9 us).
+// - many: the push in place, a thread per particle, then the plain sort.
+//   There the second gather costs more than the traffic it saves (4096
+//   cells, 524,288 particles, modes 0..2: 49.9 us in the two-pass form
+//   against 48 us; 2 x 131,072 particles, modes 0..4: 50.6 against 38 us).
 // ---------------------------------------------------------------------------
 struct PushArgs {
     int nr, ld, nm;
-    int64_t nslots;
     double idr, edge, qtmh, dt, qbm;
     double clamp;        // expansion-factor clamp of a sub-cycled push (0: none)
-    double *x1, *x2, *p1, *p2, *p3, *gamma;
-    const double *psi;   // interpolated psi (standard pusher)
-    const int32_t *cs;
-    uint32_t *key;
-    const double *eb;   // the packed E and B of the slice
+    const double *eb;    // the packed E and B of the slice
     const double *ar, *ai, *arg, *aig;   // laser envelope and gradients (PGC)
+    double *x1, *x2, *p1, *p2, *p3, *gamma;   // pushed in place (many particles)
+    SortArgs s;
 };
 
 // the arguments of every species of one launch (workgroup rows by species)
@@ -1374,17 +1382,17 @@ struct PushMulti {
 // PGC: push_u_robust_pgc_part2d / push_u_std_pgc_part2d (:1967-2219, the
 // same steps): the standard normalisation, the ponderomotive term in E with
 // the stored gamma, and the new gamma with gam_corr extrapolated half a step
-// in xi (the envelope's xi gradient)
-template <int M, bool STD, bool PGC = false>
-__global__ __launch_bounds__(256) void k_push(const PushMulti m)
+// in xi (the envelope's xi gradient).  in(f): the particle's values in the
+// order of SortArgs::s (x1, x2, p1, p2, p3, q, gamma, psi).
+struct Pushed {
+    double x1, x2, p1, p2, p3, gamma;
+};
+
+template <int M, bool STD, bool PGC, class L>
+__device__ __forceinline__ Pushed push_particle(const PushArgs &a, const L &in)
 {
-    const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= a.nslots) return;
-    const int npp = a.cs[a.nr];
-    if (p >= npp) return;
     const int nm = a.nm, ld = a.ld;
-    double x1 = a.x1[p], x2 = a.x2[p];
+    double x1 = in(0), x2 = in(1);
     double r = radius(x1, x2);
     const double pc = x1 / r, ps = x2 / r;
     double pos = __dmul_rn(r, a.idr);
@@ -1412,7 +1420,7 @@ __global__ __launch_bounds__(256) void k_push(const PushMulti m)
         la.apig[0] = t;
         const double qbm2_hf = a.qbm * a.qbm * 0.5;
         gam_corr = qbm2_hf * (la.apr * la.apr + la.api * la.api);
-        const double tmp = 0.5 * a.qbm / a.gamma[p];
+        const double tmp = 0.5 * a.qbm / in(6);
         ep[0] = ep[0] - tmp * (la.apr * la.aprg[0] + la.api * la.apig[0]);
         ep[1] = ep[1] - tmp * (la.apr * la.aprg[1] + la.api * la.apig[1]);
         ep[2] = ep[2] + tmp * (la.apr * la.aprg[2] + la.api * la.apig[2]);
@@ -1421,11 +1429,11 @@ __global__ __launch_bounds__(256) void k_push(const PushMulti m)
         apr_z = la.aprg[2];
         api_z = la.apig[2];
     }
-    double pp[3] = {a.p1[p], a.p2[p], a.p3[p]}, ut[3];
+    double pp[3] = {in(2), in(3), in(4)}, ut[3];
     double qtmh1, qtmh2;
     if constexpr (STD || PGC) {
-        qtmh1 = a.qtmh / (1.0 - a.qbm * a.psi[p]);
-        qtmh2 = qtmh1 * a.gamma[p];
+        qtmh1 = a.qtmh / (1.0 - a.qbm * in(7));
+        qtmh2 = qtmh1 * in(6);
     } else {
         const double gam = sqrt(1.0 + pp[0] * pp[0] + pp[1] * pp[1] + pp[2] * pp[2]);
         qtmh1 = a.qtmh / (gam - pp[2]);
@@ -1476,13 +1484,89 @@ __global__ __launch_bounds__(256) void k_push(const PushMulti m)
     double dtc = a.dt / (g2 - pp[2]);
     x1 = x1 + pp[0] * dtc;
     x2 = x2 + pp[1] * dtc;
-    a.p1[p] = pp[0];
-    a.p2[p] = pp[1];
-    a.p3[p] = pp[2];
-    a.gamma[p] = g2;
-    a.x1[p] = x1;
-    a.x2[p] = x2;
-    a.key[p] = cell_key(x1, x2, a.idr, a.edge, a.nr);
+    Pushed o;
+    o.x1 = x1;
+    o.x2 = x2;
+    o.p1 = pp[0];
+    o.p2 = pp[1];
+    o.p3 = pp[2];
+    o.gamma = g2;
+    return o;
+}
+
+// a particle's values where the pusher asks for them, and loaded beforehand
+struct LoadAt {
+    const SortArgs &s;
+    int64_t p;
+    __device__ __forceinline__ double operator()(int f) const { return s.s[f][p]; }
+};
+struct Loaded {
+    double v[8];
+    __device__ __forceinline__ double operator()(int f) const { return v[f]; }
+};
+
+template <int M, bool STD, bool PGC>
+__global__ __launch_bounds__(kDirectChunk) void k_push_keys(const PushMulti m)
+{
+    const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
+    if ((int)blockIdx.x >= a.s.nchunks) return;
+    extern __shared__ int lds[];
+    const int live = a.s.cs[a.nr];
+    const int64_t p = sort_element<kDirectChunk, 1>(0);
+    const Pushed o = push_particle<M, STD, PGC>(a, LoadAt{a.s, min(p, a.s.n - 1)});
+    const uint32_t kv[1] = {p < live ? cell_key(o.x1, o.x2, a.idr, a.edge, a.nr) : (uint32_t)a.nr};
+    if (p < a.s.n) a.s.key_w[p] = kv[0];
+    chunk_hist<kDirectChunk, 1>(a.s, kv, lds);
+}
+
+template <int M, bool STD, bool PGC>
+__global__ __launch_bounds__(kDirectChunk) void k_push_scatter(const PushMulti m)
+{
+    const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
+    if ((int)blockIdx.x > a.s.nchunks) return;
+    extern __shared__ int lds[];
+    // the particle's loads are issued before the counting, which hides them
+    const int64_t e = max(min(sort_element<kDirectChunk, 1>(0), a.s.n - 1), (int64_t)0);
+    const uint32_t kv[1] = {min(a.s.key[e], (uint32_t)a.nr)};
+    Loaded in;
+#pragma unroll
+    for (int f = 0; f < 8; f++) in.v[f] = a.s.s[f][e];
+    const int32_t id = a.s.sid[e];
+    int dp[1];
+    if (!scatter_positions<kDirectChunk, 1>(a.s, kv, lds, dp)) return;
+    const int at = dp[0];
+    if (at < 0) return;
+    const Pushed o = push_particle<M, STD, PGC>(a, in);
+    a.s.d[0][at] = o.x1;
+    a.s.d[1][at] = o.x2;
+    a.s.d[2][at] = o.p1;
+    a.s.d[3][at] = o.p2;
+    a.s.d[4][at] = o.p3;
+    a.s.d[5][at] = in.v[5];
+    a.s.d[6][at] = o.gamma;
+    a.s.d[7][at] = in.v[7];
+    a.s.did[at] = id;
+}
+
+template <int M, bool STD, bool PGC>
+__global__ __launch_bounds__(256) void k_push(const PushMulti m)
+{
+    const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= a.s.n) return;
+    const int npp = a.s.cs[a.nr];
+    if (p >= npp) {
+        a.s.key_w[p] = (uint32_t)a.nr;
+        return;
+    }
+    const Pushed o = push_particle<M, STD, PGC>(a, LoadAt{a.s, p});
+    a.p1[p] = o.p1;
+    a.p2[p] = o.p2;
+    a.p3[p] = o.p3;
+    a.gamma[p] = o.gamma;
+    a.x1[p] = o.x1;
+    a.x2[p] = o.x2;
+    a.s.key_w[p] = cell_key(o.x1, o.x2, a.idr, a.edge, a.nr);
 }
 
 static PushArgs push_args(qpad_ctx *c, int s)
@@ -1492,68 +1576,89 @@ static PushArgs push_args(qpad_ctx *c, int s)
     a.nr = c->g.nr;
     a.ld = c->g.ld;
     a.nm = c->g.nm;
-    a.nslots = sp.npp;
     a.idr = 1.0 / c->g.dr;
     a.edge = (double)c->g.nr * c->g.dr;
     a.qtmh = sp.qbm * c->dt2d * 0.5;
     a.dt = c->dt2d;
     a.clamp = c->clamp2d;
     a.qbm = sp.qbm;
-    a.x1 = sp.x1; a.x2 = sp.x2; a.p1 = sp.p1; a.p2 = sp.p2; a.p3 = sp.p3; a.gamma = sp.gamma;
-    a.psi = sp.psi;
-    a.cs = sp.cell_start;
-    a.key = sp.key;
     a.eb = c->eb;
     a.ar = c->f[QPAD_F_AR];
     a.ai = c->f[QPAD_F_AI];
     a.arg = c->f[QPAD_F_AR_GRAD];
     a.aig = c->f[QPAD_F_AI_GRAD];
+    a.x1 = sp.x1; a.x2 = sp.x2; a.p1 = sp.p1; a.p2 = sp.p2; a.p3 = sp.p3; a.gamma = sp.gamma;
+    a.s = sort_args(c, s);
     return a;
 }
 
-// the species of list entries in one launch (species without particles get
-// idle rows), all of the push type STD, PGC names
+// the species of list entries (all of the push type STD, PGC names and all
+// in one sort form)
 template <bool STD, bool PGC>
-static int launch_push_list(qpad_ctx *c, const int *list, int n)
+static int launch_move_list(qpad_ctx *c, const int *list, int n, bool direct)
 {
     PushMulti m;
+    SortMulti sm;
     memset(&m, 0, sizeof(m));
+    memset(&sm, 0, sizeof(sm));
+    int maxc = 0;
     int64_t nmax = 0;
     for (int i = 0; i < n; i++) {
         m.s[i] = push_args(c, list[i]);
-        nmax = std::max(nmax, c->sp[list[i]].npp);
+        sm.s[i] = m.s[i].s;
+        maxc = std::max(maxc, m.s[i].s.nchunks);
+        nmax = std::max(nmax, m.s[i].s.n);
     }
-    if (nmax == 0) return 0;
-    dim3 grid((unsigned)((nmax + 255) / 256), (unsigned)n), blk(256);
+    const int nb = c->g.nr + 1;
+    const dim3 cg(maxc, n), mg(maxc + 1, n), blk(kDirectChunk), pg((unsigned)((nmax + 255) / 256), n);
+    const size_t clds = sizeof(int) * (size_t)nb, mlds = scatter_lds<kDirectChunk>(nb, true);
     hipEvent_t stop = nullptr;
     time_begin(c, 1, &stop);
+#define QPAD_MOVE(MM)                                                                                    \
+    do {                                                                                                 \
+        if (direct) {                                                                                    \
+            if (maxc) hipLaunchKernelGGL((k_push_keys<MM, STD, PGC>), cg, blk, clds, c->stream, m);       \
+            hipLaunchKernelGGL((k_push_scatter<MM, STD, PGC>), mg, blk, mlds, c->stream, m);              \
+        } else {                                                                                         \
+            hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(256), 0, c->stream, m);                   \
+        }                                                                                                \
+    } while (0)
     switch (c->g.M) {
-    case 0: hipLaunchKernelGGL((k_push<0, STD, PGC>), grid, blk, 0, c->stream, m); break;
-    case 1: hipLaunchKernelGGL((k_push<1, STD, PGC>), grid, blk, 0, c->stream, m); break;
-    case 2: hipLaunchKernelGGL((k_push<2, STD, PGC>), grid, blk, 0, c->stream, m); break;
-    case 3: hipLaunchKernelGGL((k_push<3, STD, PGC>), grid, blk, 0, c->stream, m); break;
-    default: hipLaunchKernelGGL((k_push<4, STD, PGC>), grid, blk, 0, c->stream, m); break;
+    case 0: QPAD_MOVE(0); break;
+    case 1: QPAD_MOVE(1); break;
+    case 2: QPAD_MOVE(2); break;
+    case 3: QPAD_MOVE(3); break;
+    default: QPAD_MOVE(4); break;
     }
+#undef QPAD_MOVE
     QPAD_HIP_CHECK(hipGetLastError());
     time_end(c, 1, stop);
+    if (!direct) QPAD_TRY(launch_sort_list(c, sm, n));
+    for (int i = 0; i < n; i++) sort_swap(c->sp[list[i]]);
     return 0;
 }
 
-// species s0 .. s1-1: one launch per push present (the two PGC pushers
-// push alike)
-static int launch_push_range(qpad_ctx *c, int s0, int s1)
+// species s0 .. s1-1: one set of launches per push (the two PGC pushers push
+// alike) and sort form present
+static int launch_move_range(qpad_ctx *c, int s0, int s1)
 {
-    int list[3][kMaxSpecies], n[3] = {0, 0, 0};
-    for (int s = s0; s < s1; s++) {
-        const int g = std::min(push_group(c->sp[s].cfg.push_type), 2);
-        list[g][n[g]++] = s;
-    }
-    int rc = 0;
-    if (n[0]) rc = launch_push_list<false, false>(c, list[0], n[0]);
-    if (!rc && n[1]) rc = launch_push_list<true, false>(c, list[1], n[1]);
-    if (!rc && n[2]) rc = launch_push_list<false, true>(c, list[2], n[2]);
-    return rc;
+    for (int g = 0; g < 3; g++)
+        for (int direct = 0; direct < 2; direct++) {
+            int list[kMaxSpecies], n = 0;
+            for (int s = s0; s < s1; s++)
+                if (std::min(push_group(c->sp[s].cfg.push_type), 2) == g && sort_args(c, s).direct == direct)
+                    list[n++] = s;
+            if (!n) continue;
+            if (g == 0) QPAD_TRY((launch_move_list<false, false>(c, list, n, direct)));
+            else if (g == 1) QPAD_TRY((launch_move_list<true, false>(c, list, n, direct)));
+            else QPAD_TRY((launch_move_list<false, true>(c, list, n, direct)));
+        }
+    return 0;
 }
+
+int launch_move(qpad_ctx *c, int s) { return launch_move_range(c, s, s + 1); }
+
+int launch_move_all(qpad_ctx *c) { return launch_move_range(c, 0, c->nspecies); }
 
 // ---------------------------------------------------------------------------
 // interp_psi_part2d (part2d_class.f03:2264-2305): the field psi at every
@@ -1631,10 +1736,6 @@ int launch_interp_psi(qpad_ctx *c, int s)
     QPAD_HIP_CHECK(hipGetLastError());
     return 0;
 }
-
-int launch_push(qpad_ctx *c, int s) { return launch_push_range(c, s, s + 1); }
-
-int launch_push_all(qpad_ctx *c) { return c->nspecies ? launch_push_range(c, 0, c->nspecies) : 0; }
 
 // q_spe += qn (the neutralising background of species s)
 __global__ void k_axpy(double *y, const double *x, int64_t n)

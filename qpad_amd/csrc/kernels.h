@@ -44,7 +44,6 @@ int launch_pack_eb(qpad_ctx *c);
 // J_perp predictor for the next slice
 int launch_epilogue(qpad_ctx *c, int j);
 int slice_kernels_init();
-int sort_kernels_init();   // LDS limit of the sort scatter (k_sort.hip)
 // start of a slice after the charge deposit: q_spe and the right-hand
 // sides, the psi, Bz and Ez solves (none reads B_perp), then the
 // iteration's seed into b_spe (seed, or null to keep b_spe), 'record', b
@@ -80,7 +79,6 @@ int inject_scan_bytes(int64_t n, size_t *bytes);
 // cell_start[c] = lower bound of c in the sorted keys, c = 0 .. ncs-1
 int launch_cell_start(qpad_ctx *c, const uint32_t *key, int64_t n, int ncs, int32_t *cs);
 int launch_sort(qpad_ctx *c, int sp);            // sort by key, permute, cell starts
-int launch_sort_all(qpad_ctx *c);                // the same for every species in one set of launches
 int launch_keys(qpad_ctx *c, int sp);            // keys of the current positions
 int launch_qdeposit(qpad_ctx *c, int sp);        // per-cell partials of rho - Jz
 int launch_qdeposit_range(qpad_ctx *c, int s0, int s1);   // species s0 .. s1-1 in one launch
@@ -106,9 +104,10 @@ int launch_amjdeposit_all(qpad_ctx *c, int l, bool store_diag, bool timed, bool 
 // convergence maximum pair each; at most kConvMaxBlocks)
 constexpr int kBfThreads = 64;
 inline int conv_blocks(int nr) { return (nr + 2 + kBfThreads - 1) / kBfThreads; }
-int launch_push(qpad_ctx *c, int sp);            // push_u + push_x + keys
+// push_u + push_x and the re-sort by the new cells (from the packed fields)
+int launch_move(qpad_ctx *c, int sp);
+int launch_move_all(qpad_ctx *c);                // every species, one set of launches per pusher
 int launch_interp_psi(qpad_ctx *c, int sp);      // psi at the particles (standard pusher only)
-int launch_push_all(qpad_ctx *c);                // the same for every species in one launch
 int launch_add_qn_into_qspe(qpad_ctx *c, int sp);
 // per-species charge (species2d%q, cbq): q of species sp from its charge
 // deposit partials (at the slice start, before the current deposit reuses

@@ -231,7 +231,7 @@ static void species_free(Species &sp)
     dfree(sp.gamma); dfree(sp.psi); dfree(sp.id);
     dfree(sp.a_x1); dfree(sp.a_x2); dfree(sp.a_p1); dfree(sp.a_p2); dfree(sp.a_p3); dfree(sp.a_q);
     dfree(sp.a_gamma); dfree(sp.a_psi); dfree(sp.a_id);
-    dfree(sp.key); dfree(sp.key_alt);
+    dfree(sp.key);
     dfree(sp.cell_start); dfree(sp.qn); dfree(sp.P0); dfree(sp.P1);
     dfree(sp.ov_start); dfree(sp.ov_desc); dfree(sp.O0); dfree(sp.O1);
     dfree(sp.hist); dfree(sp.tot);
@@ -390,7 +390,7 @@ int qpad_create(const qpad_grid *gr, qpad_ctx **out)
     if (lds_need + 1024 > prop.sharedMemPerBlock)
         return fail(QPAD_E_INVALID, "nr too large for this device's LDS");
 
-    if (field_kernels_init(lds_need) != 0 || slice_kernels_init() != 0 || sort_kernels_init() != 0)
+    if (field_kernels_init(lds_need) != 0 || slice_kernels_init() != 0)
         return QPAD_E_HIP;
     TRY(noalloc_init_device(dev));
     qpad_ctx *c = new qpad_ctx{};
@@ -596,7 +596,6 @@ static int species_create(qpad_ctx *c, const qpad_species_cfg *cfg, const qpad_n
     if (!rc) rc = dalloc(&sp.id, n);
     if (!rc) rc = dalloc(&sp.a_id, n);
     if (!rc) rc = dalloc(&sp.key, n);
-    if (!rc) rc = dalloc(&sp.key_alt, n);
     if (!rc) rc = dalloc(&sp.cell_start, (size_t)c->g.nr + 2);
     if (!rc) rc = dalloc(&sp.qn, f1_size(c, 1));
     if (!rc) rc = dalloc(&sp.P0, (size_t)c->g.nr * 8 * c->g.nm);
@@ -1078,8 +1077,7 @@ static int slice_finish(qpad_ctx *c, SliceRun &st)
         TRY(launch_iter_fold(c, false));
         for (int s = 0; s < c->nspecies; s++)
             if (c->sp[s].neutral) TRY(launch_neutral_update(c, s));
-        TRY(launch_push_all(c));
-        TRY(launch_sort_all(c));
+        TRY(launch_move_all(c));
         st.sub++;
         return subcycle_start(c, st);
     }
@@ -1101,8 +1099,7 @@ static int slice_finish(qpad_ctx *c, SliceRun &st)
     }
     const bool net = seednet_active(c);
     if (net) TRY(seednet_mark(c));
-    TRY(launch_push_all(c));
-    TRY(launch_sort_all(c));
+    TRY(launch_move_all(c));
     if (net) TRY(seednet_after_epilogue(c, j, (st.overlap && j < c->g.nxi) ? j + 1 : 0, true));
     c->dt2d = c->g.dxi;
     c->clamp2d = 0.0;
@@ -1401,11 +1398,10 @@ static int species_push(qpad_ctx *c, int32_t s, double dxi, double clamp)
     TRY(launch_pack_eb(c));
     c->dt2d = dxi;
     c->clamp2d = clamp;
-    int rc = launch_push(c, s);
+    int rc = launch_move(c, s);
     c->dt2d = c->g.dxi;
     c->clamp2d = 0.0;
     TRY(rc);
-    TRY(launch_sort(c, s));
     return sync(c);
 }
 

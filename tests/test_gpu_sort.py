@@ -1,0 +1,62 @@
+"""The re-sort by radial cell at the sizes where its forms meet: one
+particle, chunk edges of both chunk shapes (512 and 2048), the most particles
+of the form without a scan launch (16384) and one more, cell counts on both
+sides of the rank window and of the bins that form keeps in LDS.  Particles
+handed over in random order spread every chunk over all cells (the ranks taken
+in turn), nearly sorted ones stay within the window; some lie outside the box
+and are removed.  The order is exact: by cell, then by the order given."""
+import numpy as np
+import pytest
+
+from qpad_amd import Simulation, configs
+
+pytestmark = pytest.mark.gpu
+
+
+def _ppc(n, nr):
+    # species large enough for n particles (npmax = 2 x injected)
+    return (1, max(1, -(-n // (2 * nr))))
+
+
+@pytest.mark.parametrize("nr,n", [(40, 1), (40, 511), (40, 513), (600, 4096), (1100, 16384), (1100, 16385),
+                                  (2100, 2049), (4200, 9000), (4200, 70001)])
+@pytest.mark.parametrize("spread", [False, True])
+def test_sort_is_stable_and_complete(nr, n, spread):
+    sim = Simulation(configs.small(nr=nr, nxi=2, max_mode=0, ppc=_ppc(n, nr), total_num=16))
+    g = sim.grid
+    rng = np.random.default_rng(n + nr)
+    cell = rng.integers(0, nr + max(nr // 20, 1), n)          # some past the last cell: removed
+    if not spread:
+        cell = np.sort(cell) + rng.integers(-3, 4, n)
+        cell = np.clip(cell, 0, None)
+    r = (cell + rng.uniform(0.1, 0.9, n)) * g.dr
+    ph = rng.uniform(0.0, 2.0 * np.pi, n)
+    z = np.zeros(n)
+    ids = np.arange(n, dtype=np.int32)
+    sim.spe[0].set({"x1": r * np.cos(ph), "x2": r * np.sin(ph), "p1": 1.0 * ids, "p2": z, "p3": z, "q": -1.0 - ids,
+                    "gamma": z + 1.0, "psi": 0.5 * ids, "id": ids})
+    got = sim.spe[0].get()
+    order = np.argsort(cell, kind="stable")
+    order = order[cell[order] < nr]
+    assert np.array_equal(got["id"], ids[order])
+    for k, v in (("x1", r * np.cos(ph)), ("p1", 1.0 * ids), ("q", -1.0 - ids), ("psi", 0.5 * ids)):
+        assert np.array_equal(got[k], v[order]), k
+    sim.close()
+
+
+@pytest.mark.parametrize("ppc,direct", [((2, 16), True), ((4, 130), False)])
+def test_push_forms_keep_the_sorted_order(ppc, direct):
+    """both push forms leave the particles grouped by cell, each cell in the
+    order its particles had before (no particle lost or doubled)"""
+    sim = Simulation(configs.small(nr=64, nxi=40, max_mode=1, ppc=ppc, total_num=1 << 12, offset_x=0.02))
+    assert (64 * ppc[0] * ppc[1] <= 16384) == direct
+    sim.step3d_begin()
+    n0 = sim.spe[0].count()
+    for j in range(1, 31):
+        sim.slice(j)
+    p = sim.spe[0].get()
+    c = np.floor(np.hypot(p["x1"], p["x2"]) / sim.grid.dr).astype(int)
+    assert np.all(np.diff(c) >= 0) and c.max() < 64
+    assert len(np.unique(p["id"])) == len(p["id"]) <= n0
+    assert np.all(np.isfinite(p["gamma"])) and np.max(np.abs(p["p1"])) > 1e-3
+    sim.close()
