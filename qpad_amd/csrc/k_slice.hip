@@ -44,7 +44,6 @@ struct SrcArgs {
     // overflow rows of crowded cells (cell_partial)
     const double *O0[kMaxSpecies], *O1[kMaxSpecies];
     const int32_t *os[kMaxSpecies];
-    int ns;
     double *cu_out, *acu_out, *amu_out, *dcu;
     const double *b_spe;
     double *src;
@@ -57,16 +56,23 @@ struct SrcArgs {
 constexpr int kSrcTile = 16;
 constexpr int kSrcHalo = 2;
 constexpr int kSrcTL = kSrcTile + 2 * kSrcHalo;
-static_assert(kSrcTile * (kMaxMode + 1) <= 256, "one B+/B- item per k_src thread");
+
+// waves of a k_src workgroup: the tile's B+/B- items (a thread per node and
+// mode), then three groups (a thread per node and mode array): Bz sources,
+// Ez sources, and the copies out
+constexpr int src_bpm_waves(int M) { return (kSrcTile * (M + 1) + 63) / 64; }
+constexpr int src_k_waves(int M) { return (kSrcTile * (2 * M + 1) + 63) / 64; }
+constexpr int src_threads(int M) { return 64 * (src_bpm_waves(M) + 3 * src_k_waves(M)); }
 
 // cu (base 0), acu (3) or amu (5) of the tile in LDS as [comp8][k][j],
 // j = i - (i0 - 2)
+template <int NM, int BASE>
 struct TileArr {
     const double *s;
-    int nm, base, i0;
+    int i0;
     __device__ __forceinline__ double operator()(int c, int k, int i) const
     {
-        return s[((size_t)(base + c) * nm + k) * kSrcTL + (i - i0 + kSrcHalo)];
+        return s[((BASE + c) * NM + k) * kSrcTL + (i - i0 + kSrcHalo)];
     }
 };
 
@@ -74,16 +80,10 @@ struct TileArr {
 // every species, with the axis rules and 1/r of amjdeposit_robust_part2d
 // (part2d_class.f03:914-1004).  P0[cell][v] is the deposit of cell `cell`
 // on its inner node, P1 on its outer node, v = comp8 * nm + k.  Split in an
-// address step (clamped, so the loads are always valid) and a combine step.
-__device__ __forceinline__ void partial_addr(const FieldCommon &g, int comp, int k, int i, int &cell0,
-                                             int &cell1, size_t &c0, size_t &c1)
-{
-    const int nm = g.nm, nr = g.nr, NV = 8 * nm, v = comp * nm + k;
-    cell0 = min(max(i - 1, 0), nr - 1);
-    cell1 = min(max(i - 2, 0), nr - 1);
-    c0 = (size_t)cell0 * NV + v;
-    c1 = (size_t)cell1 * NV + v;
-}
+// address step (clamped cells, so the loads are always valid) and a combine
+// step.
+__device__ __forceinline__ int inner_cell(int nr, int i) { return min(max(i - 1, 0), nr - 1); }
+__device__ __forceinline__ int outer_cell(int nr, int i) { return min(max(i - 2, 0), nr - 1); }
 
 template <int NS>
 __device__ __forceinline__ double combine_node(int nr, int comp, int k, int i, const double (&d0)[NS],
@@ -128,17 +128,26 @@ struct BspeNode {
 };
 
 // one workgroup per tile of kSrcTile nodes: (1) cu, acu, amu of the tile
-// and its halo into LDS; (2) B+/B- sources of every mode and dJ/dxi at the
-// tile's nodes 1..nr; (3) cu, acu, amu out (nodes 0..nr+1) and the Bz and Ez
-// sources of every mode array
-template <int NS>
-__global__ __launch_bounds__(256) void k_src(SrcArgs a)
+// and its halo into LDS; (2) by wave: B+/B- sources of every mode and dJ/dxi
+// at the tile's nodes 1..nr; Bz sources; Ez sources; cu, acu, amu out (nodes
+// 0..nr+1).  A chain of a few loads and divisions: the mode count is a
+// template parameter so that a thread holds exactly its entries of the tile
+// and their indices need no division, and the four kinds of items run on
+// waves of their own (mean launch, those after convergence included, against
+// one kernel for every mode count with the items in turn: 256 nodes, M = 1
+// 5.7 -> 3.7 us; 512 nodes, M = 0 4.1 -> 2.7 us; hosing deck, M = 4 and two
+// species 7.7 -> 5.0 us)
+template <int NS, int M>
+__global__ __launch_bounds__(src_threads(M)) void k_src(SrcArgs a)
 {
-    extern __shared__ double tile[];
+    constexpr int NM = 2 * M + 1, NV = 8 * NM, T = src_threads(M), kEntries = NV * kSrcTL;
+    constexpr int U = (kEntries + T - 1) / T;   // entries per thread, loaded together
+    constexpr int kBpm = 64 * src_bpm_waves(M), kPerK = 64 * src_k_waves(M);
+    __shared__ double tile[kEntries];
     // the converged flag: with adaptive queuing (late_done) almost every
-    // launch works, and the flag is tested after the first pass's loads are
-    // issued (one round trip less); with fixed queuing about half the
-    // launches come after convergence and return before loading anything
+    // launch works, and the flag is tested after the loads are issued (one
+    // round trip less); with fixed queuing about half the launches come after
+    // convergence and return before loading anything
     // (a vector load, through an offset the compiler cannot see is zero: its
     // wait does not also wait for the kernel-argument scalar loads, and it
     // retires before the data loads issued after it)
@@ -148,15 +157,14 @@ __global__ __launch_bounds__(256) void k_src(SrcArgs a)
         if (__builtin_amdgcn_readfirstlane(done)) return;
     }
     const FieldCommon &g = a.g;
-    const int nm = g.nm, ld = g.ld, nr = g.nr, M = g.M;
-    const int t = threadIdx.x, T = blockDim.x;
+    const int nm = NM, ld = g.ld, nr = g.nr;
+    const int t = threadIdx.x;
     const int i0 = blockIdx.x * kSrcTile;
-    const int n_tile = 8 * nm * kSrcTL;
     // does any cell the tile reads have overflow rows (crowded cells)?  The
-    // test is uniform over the workgroup and is only needed after the
-    // pass's loads are issued.  Such tiles take a lean path (one entry at a
-    // time, each cell's overflow rows added in row order), so that the
-    // common path keeps its registers and occupancy.
+    // test is uniform over the workgroup and is only needed after the loads
+    // are issued.  Such tiles take a lean path (one entry at a time, each
+    // cell's overflow rows added in row order), so that the common path keeps
+    // its registers and occupancy.
     const int lo = max(i0 - kSrcHalo - 2, 0), hi = min(i0 + kSrcTile + kSrcHalo - 2, nr - 1);
     int os_lo[NS], os_hi[NS];
 #pragma unroll
@@ -165,74 +173,30 @@ __global__ __launch_bounds__(256) void k_src(SrcArgs a)
         os_hi[q] = a.os[q][hi + 1];
     }
     // b_spe at the node of this thread's B+/B- item (the only b_spe values
-    // the sources read), requested first; one item per thread
-    // (kSrcTile * (kMaxMode + 1) <= 256 threads)
+    // the sources read), requested first
     const int m2 = t / kSrcTile, i2 = i0 + t % kSrcTile;
     const bool item2 = t < kSrcTile * (M + 1) && i2 >= 1 && i2 <= nr;
     const int kr2 = m2 == 0 ? 0 : 2 * m2 - 1, ki2 = m2 == 0 ? 0 : 2 * m2;
     const int i2c = min(max(i2, 1), nr);
     const BspeNode bn{kr2, FX(a.b_spe, 0, min(kr2, nm - 1), i2c), FX(a.b_spe, 1, min(kr2, nm - 1), i2c),
                       FX(a.b_spe, 0, min(ki2, nm - 1), i2c), FX(a.b_spe, 1, min(ki2, nm - 1), i2c)};
-    const int NV = 8 * nm;
-    // 8 entries per thread per pass so that their loads are in flight
-    // together; entry idx = j * NV + v (node j of the tile, value v), so that
+    // entry idx = j * NV + v (node j of the tile, value v), so that
     // neighbouring threads read neighbouring values of one cell's partial row
     // (coalesced) and the tile in LDS is [v][j]
-    double d0[8][NS], d1[8][NS];
-    auto pass_loads = [&](int base) {
+    double d0[U][NS], d1[U][NS];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int idx = min(base + u * T, n_tile - 1);
-            const int j = idx / NV, vv = idx - j * NV, comp = vv / nm, k = vv - comp * nm;
-            const int i = min(max(i0 - kSrcHalo + j, 0), nr + 1);
-            int cl0, cl1;
-            size_t c0, c1;
-            partial_addr(g, comp, k, i, cl0, cl1, c0, c1);
+    for (int u = 0; u < U; u++) {
+        const int idx = min(t + u * T, kEntries - 1);
+        const int j = idx / NV, vv = idx % NV, i = min(max(i0 - kSrcHalo + j, 0), nr + 1);
+        const size_t c0 = (size_t)inner_cell(nr, i) * NV + vv, c1 = (size_t)outer_cell(nr, i) * NV + vv;
 #pragma unroll
-            for (int q = 0; q < NS; q++) {
-                d0[u][q] = a.P0[q][c0];
-                d1[u][q] = a.P1[q][c1];
-            }
+        for (int q = 0; q < NS; q++) {
+            d0[u][q] = a.P0[q][c0];
+            d1[u][q] = a.P1[q][c1];
         }
-    };
-    auto pass_combine = [&](int base, bool ovf) {
-        if (!ovf) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int idx = base + u * T;
-                if (idx >= n_tile) break;
-                const int j = idx / NV, vv = idx - j * NV, comp = vv / nm, k = vv - comp * nm;
-                const int i = i0 - kSrcHalo + j;
-                const double v = combine_node<NS>(nr, comp, k, min(max(i, 0), nr + 1), d0[u], d1[u]);
-                tile[vv * kSrcTL + j] = (i >= 0 && i <= nr + 1) ? v : 0.0;
-            }
-        } else {
-#pragma unroll 1
-            for (int u = 0; u < 8; u++) {
-                const int idx = base + u * T;
-                if (idx >= n_tile) break;
-                const int j = idx / NV, vv = idx - j * NV, comp = vv / nm, k = vv - comp * nm;
-                const int i = i0 - kSrcHalo + j;
-                const int ic = min(max(i, 0), nr + 1);
-                int cl0, cl1;
-                size_t c0, c1;
-                partial_addr(g, comp, k, ic, cl0, cl1, c0, c1);
-                double e0[NS], e1[NS];
-#pragma unroll
-                for (int q = 0; q < NS; q++) {
-                    e0[q] = add_rows(a.P0[q][c0], a.O0[q], a.os[q][cl0], a.os[q][cl0 + 1], NV, vv);
-                    e1[q] = add_rows(a.P1[q][c1], a.O1[q], a.os[q][cl1], a.os[q][cl1 + 1], NV, vv);
-                }
-                const double val = combine_node<NS>(nr, comp, k, ic, e0, e1);
-                tile[vv * kSrcTL + j] = (i >= 0 && i <= nr + 1) ? val : 0.0;
-            }
-        }
-    };
-    // first pass peeled (a loop header would wait for every load in flight,
-    // the b_spe requests above included, before this pass's loads)
-    pass_loads(t);
+    }
     // (the empty asms keep the compiler from hoisting the tests, and the
-    // wait for their loads, above this pass's loads)
+    // wait for their loads, above the loads)
     if (a.late_done) {
         __asm__ volatile("" : "+v"(done));
         if (__builtin_amdgcn_readfirstlane(done)) return;
@@ -244,15 +208,40 @@ __global__ __launch_bounds__(256) void k_src(SrcArgs a)
         __asm__ volatile("" : "+v"(l_), "+v"(h_));
         ovf = ovf || __builtin_amdgcn_readfirstlane(h_) != __builtin_amdgcn_readfirstlane(l_);
     }
-    pass_combine(t, ovf);
-    for (int base = t + 8 * T; base < n_tile; base += 8 * T) {
-        pass_loads(base);
-        pass_combine(base, ovf);
+    if (!ovf) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int idx = t + u * T;
+            if (idx >= kEntries) break;
+            const int j = idx / NV, vv = idx % NV, i = i0 - kSrcHalo + j;
+            const double v = combine_node<NS>(nr, vv / NM, vv % NM, min(max(i, 0), nr + 1), d0[u], d1[u]);
+            tile[vv * kSrcTL + j] = (i >= 0 && i <= nr + 1) ? v : 0.0;
+        }
+    } else {
+#pragma unroll 1
+        for (int idx = t; idx < kEntries; idx += T) {
+            const int j = idx / NV, vv = idx % NV, i = i0 - kSrcHalo + j;
+            const int ic = min(max(i, 0), nr + 1);
+            const int cl0 = inner_cell(nr, ic), cl1 = outer_cell(nr, ic);
+            double e0[NS], e1[NS];
+#pragma unroll
+            for (int q = 0; q < NS; q++) {
+                e0[q] = cell_partial(a.P0[q], a.O0[q], a.os[q], cl0, NV, vv);
+                e1[q] = cell_partial(a.P1[q], a.O1[q], a.os[q], cl1, NV, vv);
+            }
+            const double v = combine_node<NS>(nr, vv / NM, vv % NM, ic, e0, e1);
+            tile[vv * kSrcTL + j] = (i >= 0 && i <= nr + 1) ? v : 0.0;
+        }
     }
     __syncthreads();
-    const TileArr cu{tile, nm, 0, i0}, acu{tile, nm, 3, i0}, amu{tile, nm, 5, i0};
-    // B+/B- of mode m and dJ/dxi
-    if (item2) {
+    const TileArr<NM, 0> cu{tile, i0};
+    const TileArr<NM, 3> acu{tile, i0};
+    const TileArr<NM, 5> amu{tile, i0};
+    // the wave's kind of items
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (w < src_bpm_waves(M)) {
+        // B+/B- of mode m and dJ/dxi
+        if (!item2) return;
         const int m = m2, i = i2;
         const int kr = kr2, ki = 2 * m;
         double dr_[2], di_[2] = {0.0, 0.0}, bpm[4];
@@ -267,21 +256,37 @@ __global__ __launch_bounds__(256) void k_src(SrcArgs a)
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) a.src[(size_t)(4 * m + q) * nr + i - 1] = bpm[q];
+        return;
     }
-    // cu, acu, amu out; Bz and Ez sources
-    for (int it = t; it < kSrcTile * nm; it += T) {
-        const int k = it / kSrcTile, i = i0 + it % kSrcTile, m = mode_of(k);
-        if (i > nr + 1) continue;
+    const int kind = (w - src_bpm_waves(M)) / src_k_waves(M);
+    const int it = t - kBpm - kind * kPerK, k = it / kSrcTile, i = i0 + it % kSrcTile;
+    if (it >= kSrcTile * NM || i > nr + 1) return;
+    if (kind == 2) {
 #pragma unroll
         for (int c = 0; c < 3; c++) FX(a.cu_out, c, k, i) = cu(c, k, i);
 #pragma unroll
         for (int c = 0; c < 2; c++) FX(a.acu_out, c, k, i) = acu(c, k, i);
 #pragma unroll
         for (int c = 0; c < 3; c++) FX(a.amu_out, c, k, i) = amu(c, k, i);
-        if (i < 1 || i > nr) continue;
+        return;
+    }
+    if (i < 1 || i > nr) return;
+    if (kind == 0)
         a.src[(size_t)src_bz(M, k) * nr + i - 1] = bz_source(g, cu, k, i);
-        a.src[(size_t)src_ez(M, nm, k) * nr + i - 1] =
-            (m == 0) ? ez_source_0(g, cu, i) : ez_source_m(g, cu, k, i);
+    else
+        a.src[(size_t)src_ez(M, nm, k) * nr + i - 1] = (k == 0) ? ez_source_0(g, cu, i) : ez_source_m(g, cu, k, i);
+}
+
+template <int NS>
+static void launch_src_ns(const SrcArgs &s, int M, hipStream_t st)
+{
+    const dim3 grid((unsigned)((s.g.nr + 2 + kSrcTile - 1) / kSrcTile));
+    switch (M) {
+    case 0: hipLaunchKernelGGL((k_src<NS, 0>), grid, dim3(src_threads(0)), 0, st, s); break;
+    case 1: hipLaunchKernelGGL((k_src<NS, 1>), grid, dim3(src_threads(1)), 0, st, s); break;
+    case 2: hipLaunchKernelGGL((k_src<NS, 2>), grid, dim3(src_threads(2)), 0, st, s); break;
+    case 3: hipLaunchKernelGGL((k_src<NS, 3>), grid, dim3(src_threads(3)), 0, st, s); break;
+    default: hipLaunchKernelGGL((k_src<NS, 4>), grid, dim3(src_threads(4)), 0, st, s); break;
     }
 }
 
@@ -542,7 +547,6 @@ int launch_iteration_fields(qpad_ctx *c, int j, int l)
     SrcArgs s;
     memset(&s, 0, sizeof(s));
     s.g = g;
-    s.ns = c->nspecies;
     for (int q = 0; q < c->nspecies; q++) {
         s.P0[q] = c->sp[q].P0;
         s.P1[q] = c->sp[q].P1;
@@ -558,13 +562,11 @@ int launch_iteration_fields(qpad_ctx *c, int j, int l)
     s.src = c->src;
     s.it = c->it;
     s.late_done = c->adaptive;
-    const size_t src_lds = sizeof(double) * 8 * c->g.nm * kSrcTL;
-    const dim3 sgrid((unsigned)((c->g.nr + 2 + kSrcTile - 1) / kSrcTile));
     switch (c->nspecies) {
-    case 1: hipLaunchKernelGGL(k_src<1>, sgrid, dim3(256), src_lds, c->stream, s); break;
-    case 2: hipLaunchKernelGGL(k_src<2>, sgrid, dim3(256), src_lds, c->stream, s); break;
-    case 3: hipLaunchKernelGGL(k_src<3>, sgrid, dim3(256), src_lds, c->stream, s); break;
-    default: hipLaunchKernelGGL(k_src<4>, sgrid, dim3(256), src_lds, c->stream, s); break;
+    case 1: launch_src_ns<1>(s, c->g.M, c->stream); break;
+    case 2: launch_src_ns<2>(s, c->g.M, c->stream); break;
+    case 3: launch_src_ns<3>(s, c->g.M, c->stream); break;
+    default: launch_src_ns<4>(s, c->g.M, c->stream); break;
     }
     QPAD_HIP_CHECK(hipGetLastError());
 
@@ -1034,11 +1036,6 @@ static int set_lds_attr_slice()
 
 int slice_kernels_init()
 {
-    const void *srcs[] = {(const void *)k_src<1>, (const void *)k_src<2>, (const void *)k_src<3>,
-                          (const void *)k_src<4>};
-    for (const void *k : srcs)
-        QPAD_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)(sizeof(double) * 8 * kMaxNm * kSrcTL)));
     QPAD_TRY(set_lds_attr_slice<1>());
     QPAD_TRY(set_lds_attr_slice<2>());
     QPAD_TRY(set_lds_attr_slice<4>());
