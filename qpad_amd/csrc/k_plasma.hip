@@ -1350,7 +1350,7 @@ int launch_amjdeposit_all(qpad_ctx *c, int l, bool store_diag, bool timed, bool 
 // push_u_robust (part2d_class.f03:1879-1965) + push_x (:2221-2262) + the
 // re-sort by the new cells (update_bound :2307-2353 is the key nr).
 // Particles that already left the box (past cell_start[nr]) keep key nr.
-// Two forms, by the number of particles (SortArgs::direct):
+// Two forms, by the form of the sort (sort_args):
 // - few particles: two launches.  The counting pass pushes them only for
 //   their new cells, the scattering pass pushes them again on the way to their
 //   sorted places; the launches' latencies are all that counts (blowout
@@ -1506,34 +1506,34 @@ struct Loaded {
 };
 
 template <int M, bool STD, bool PGC>
-__global__ __launch_bounds__(kDirectChunk) void k_push_keys(const PushMulti m)
+__global__ __launch_bounds__(kSmallChunk) void k_push_keys(const PushMulti m)
 {
     const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     if ((int)blockIdx.x >= a.s.nchunks) return;
-    extern __shared__ int lds[];
+    extern __shared__ __attribute__((aligned(16))) int lds[];
     const int live = a.s.cs[a.nr];
-    const int64_t p = sort_element<kDirectChunk, 1>(0);
+    const int64_t p = sort_element<kSmallChunk, 1>(0);
     const Pushed o = push_particle<M, STD, PGC>(a, LoadAt{a.s, min(p, a.s.n - 1)});
     const uint32_t kv[1] = {p < live ? cell_key(o.x1, o.x2, a.idr, a.edge, a.nr) : (uint32_t)a.nr};
     if (p < a.s.n) a.s.key_w[p] = kv[0];
-    chunk_hist<kDirectChunk, 1>(a.s, kv, lds);
+    chunk_hist<kSmallChunk, 1>(a.s, kv, lds);
 }
 
 template <int M, bool STD, bool PGC>
-__global__ __launch_bounds__(kDirectChunk) void k_push_scatter(const PushMulti m)
+__global__ __launch_bounds__(kSmallChunk) void k_push_scatter(const PushMulti m)
 {
     const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     if ((int)blockIdx.x > a.s.nchunks) return;
-    extern __shared__ int lds[];
+    extern __shared__ __attribute__((aligned(16))) int lds[];
     // the particle's loads are issued before the counting, which hides them
-    const int64_t e = max(min(sort_element<kDirectChunk, 1>(0), a.s.n - 1), (int64_t)0);
+    const int64_t e = max(min(sort_element<kSmallChunk, 1>(0), a.s.n - 1), (int64_t)0);
     const uint32_t kv[1] = {min(a.s.key[e], (uint32_t)a.nr)};
     Loaded in;
 #pragma unroll
     for (int f = 0; f < 8; f++) in.v[f] = a.s.s[f][e];
     const int32_t id = a.s.sid[e];
     int dp[1];
-    if (!scatter_positions<kDirectChunk, 1>(a.s, kv, lds, dp)) return;
+    if (!scatter_positions<kSmallChunk, 1>(a.s, kv, lds, dp)) return;
     const int at = dp[0];
     if (at < 0) return;
     const Pushed o = push_particle<M, STD, PGC>(a, in);
@@ -1595,7 +1595,7 @@ static PushArgs push_args(qpad_ctx *c, int s)
 // the species of list entries (all of the push type STD, PGC names and all
 // in one sort form)
 template <bool STD, bool PGC>
-static int launch_move_list(qpad_ctx *c, const int *list, int n, bool direct)
+static int launch_move_list(qpad_ctx *c, const int *list, int n, int form)
 {
     PushMulti m;
     SortMulti sm;
@@ -1610,13 +1610,13 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, bool direct)
         nmax = std::max(nmax, m.s[i].s.n);
     }
     const int nb = c->g.nr + 1;
-    const dim3 cg(maxc, n), mg(maxc + 1, n), blk(kDirectChunk), pg((unsigned)((nmax + 255) / 256), n);
-    const size_t clds = sizeof(int) * (size_t)nb, mlds = scatter_lds<kDirectChunk>(nb, true);
+    const dim3 cg(maxc, n), mg(maxc + 1, n), blk(kSmallChunk), pg((unsigned)((nmax + 255) / 256), n);
+    const size_t clds = sizeof(int) * (size_t)nb, mlds = scatter_lds<kSmallChunk>(nb, SORT_DIRECT);
     hipEvent_t stop = nullptr;
     time_begin(c, 1, &stop);
 #define QPAD_MOVE(MM)                                                                                    \
     do {                                                                                                 \
-        if (direct) {                                                                                    \
+        if (form == SORT_DIRECT) {                                                                                    \
             if (maxc) hipLaunchKernelGGL((k_push_keys<MM, STD, PGC>), cg, blk, clds, c->stream, m);       \
             hipLaunchKernelGGL((k_push_scatter<MM, STD, PGC>), mg, blk, mlds, c->stream, m);              \
         } else {                                                                                         \
@@ -1633,7 +1633,7 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, bool direct)
 #undef QPAD_MOVE
     QPAD_HIP_CHECK(hipGetLastError());
     time_end(c, 1, stop);
-    if (!direct) QPAD_TRY(launch_sort_list(c, sm, n));
+    if (form != SORT_DIRECT) QPAD_TRY(launch_sort_list(c, sm, n));
     for (int i = 0; i < n; i++) sort_swap(c->sp[list[i]]);
     return 0;
 }
@@ -1643,15 +1643,15 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, bool direct)
 static int launch_move_range(qpad_ctx *c, int s0, int s1)
 {
     for (int g = 0; g < 3; g++)
-        for (int direct = 0; direct < 2; direct++) {
+        for (int form = 0; form < SORT_FORMS; form++) {
             int list[kMaxSpecies], n = 0;
             for (int s = s0; s < s1; s++)
-                if (std::min(push_group(c->sp[s].cfg.push_type), 2) == g && sort_args(c, s).direct == direct)
+                if (std::min(push_group(c->sp[s].cfg.push_type), 2) == g && sort_args(c, s).form == form)
                     list[n++] = s;
             if (!n) continue;
-            if (g == 0) QPAD_TRY((launch_move_list<false, false>(c, list, n, direct)));
-            else if (g == 1) QPAD_TRY((launch_move_list<true, false>(c, list, n, direct)));
-            else QPAD_TRY((launch_move_list<false, true>(c, list, n, direct)));
+            if (g == 0) QPAD_TRY((launch_move_list<false, false>(c, list, n, form)));
+            else if (g == 1) QPAD_TRY((launch_move_list<true, false>(c, list, n, form)));
+            else QPAD_TRY((launch_move_list<false, true>(c, list, n, form)));
         }
     return 0;
 }

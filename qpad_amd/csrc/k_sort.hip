@@ -27,7 +27,7 @@ __global__ __launch_bounds__(T) void k_sort_hist(const SortMulti m)
 {
     const SortArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     if ((int)blockIdx.x >= a.nchunks) return;   // the species has fewer chunks than the grid
-    extern __shared__ int lds[];
+    extern __shared__ __attribute__((aligned(16))) int lds[];
     uint32_t kv[PER];
     load_keys<T, PER>(a, kv);
     chunk_hist<T, PER>(a, kv, lds);
@@ -44,7 +44,6 @@ template <int RUN>
 __global__ __launch_bounds__(kScanThreads) void k_sort_scan(const SortMulti m)
 {
     const SortArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
-    if (a.direct) return;   // few chunks: the scattering workgroups sum the rows
     __shared__ int gsum[kScanGroups][kScanBins];
     const int t = threadIdx.x;
     const int lb = t % kScanBins, grp = t / kScanBins;
@@ -89,7 +88,7 @@ __global__ __launch_bounds__(T) void k_sort_scatter(const SortMulti m)
 {
     const SortArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     if ((int)blockIdx.x > a.nchunks) return;
-    extern __shared__ int lds[];
+    extern __shared__ __attribute__((aligned(16))) int lds[];
     uint32_t kv[PER];
     load_keys<T, PER>(a, kv);
     int dp[PER];
@@ -121,7 +120,11 @@ int sort_workspace(int64_t npmax, int nr, size_t *hist_ints)
                   std::to_string((long long)kMaxSortChunks * kSortChunk) + ")");
         return QPAD_E_INVALID;
     }
-    *hist_ints = (size_t)std::max<int64_t>(nchunks, kDirectChunks) * (size_t)(nr + 1);
+    // up to kMidMax particles in smaller chunks; the direct form's rows hold
+    // 16-bit counts, two small chunks in the space of a mid one
+    const int64_t mid = (std::min(npmax, kMidMax) + kMidChunk - 1) / kMidChunk;
+    static_assert(2 * kSmallChunk == kMidChunk, "16-bit rows of small chunks in the space of the mid ones");
+    *hist_ints = (size_t)std::max(nchunks, mid) * (size_t)hist16_row(nr + 1);
     return 0;
 }
 
@@ -133,11 +136,17 @@ SortArgs sort_args(qpad_ctx *c, int s)
     memset(&a, 0, sizeof(a));
     a.n = n;
     a.nb = c->g.nr + 1;
-    // few particles: small chunks and no scan launch (blowout deck, 4096
-    // particles in 256 cells: 5.4 + 2.9 + 2.8 + 13.0 us for push, counting,
-    // scan and scatter before; see k_push_scatter)
-    a.direct = n <= (int64_t)kDirectChunk * kDirectChunks && a.nb <= kDirectBins;
-    const int chunk = a.direct ? kDirectChunk : kSortChunk;
+    // push and re-sort, us a slice, chunks of 2048 with the scan launch -> the
+    // form now: direct 4096 particles in 256 cells 24.1 -> 11.8, 21189 in 1009
+    // 23.4 -> 16.0, 24576 in 768 27 -> 19.5 (the sum over the chunks grows with
+    // chunks x bins: at 131072 its 2 us equal the scan launch); sort alone, mid
+    // form: 65536 in 512 cells 20.0 -> 17.1; two species of 131072 in 2048
+    // 22.1 -> 22.1, where the chunk counts' traffic meets the gain
+    const int64_t small = (n + kSmallChunk - 1) / kSmallChunk;
+    if (n > kMidMax) a.form = SORT_LARGE;
+    else if (a.nb > kDirectBins || small > kDirectChunks || small * a.nb > kDirectWork) a.form = SORT_MID;
+    else a.form = SORT_DIRECT;
+    const int chunk = a.form == SORT_LARGE ? kSortChunk : a.form == SORT_MID ? kMidChunk : kSmallChunk;
     a.nchunks = (int)((n + chunk - 1) / chunk);
     a.key = sp.key;
     a.key_w = sp.key;
@@ -187,18 +196,19 @@ int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns)
     int maxc = 0;
     for (int i = 0; i < ns; i++) maxc = std::max(maxc, m.s[i].nchunks);
     const int nb = c->g.nr + 1;
-    const size_t lds = sizeof(int) * (size_t)nb;
+    const int form = m.s[0].form;
+    const size_t hl = sizeof(int) * (size_t)nb;
     const dim3 cg(std::max(maxc, 1), ns), mg(maxc + 1, ns);
-    if (m.s[0].direct) {
-        if (maxc) hipLaunchKernelGGL((k_sort_hist<kDirectChunk, 1>), cg, dim3(kDirectChunk), lds, c->stream, m);
-        hipLaunchKernelGGL((k_sort_scatter<kDirectChunk, 1>), mg, dim3(kDirectChunk), scatter_lds<kDirectChunk>(nb, true),
-                           c->stream, m);
-    } else {
-        constexpr int T = kSortChunk / 2;
-        if (maxc) hipLaunchKernelGGL((k_sort_hist<T, 2>), cg, dim3(T), lds, c->stream, m);
-        QPAD_TRY(launch_sort_scan(c, m, ns, maxc));
-        hipLaunchKernelGGL((k_sort_scatter<T, 2>), mg, dim3(T), scatter_lds<T>(nb, false), c->stream, m);
-    }
+#define QPAD_SORT(T, PER)                                                                              \
+    do {                                                                                              \
+        if (maxc) hipLaunchKernelGGL((k_sort_hist<T, PER>), cg, dim3(T), hl, c->stream, m);            \
+        if (form != SORT_DIRECT) QPAD_TRY(launch_sort_scan(c, m, ns, maxc));                           \
+        hipLaunchKernelGGL((k_sort_scatter<T, PER>), mg, dim3(T), scatter_lds<T>(nb, form), c->stream, m); \
+    } while (0)
+    if (form == SORT_LARGE) QPAD_SORT(kSortThreads, 2);
+    else if (form == SORT_MID) QPAD_SORT(kMidThreads, 2);
+    else QPAD_SORT(kSmallChunk, 1);
+#undef QPAD_SORT
     QPAD_HIP_CHECK(hipGetLastError());
     return 0;
 }

@@ -18,11 +18,13 @@
 // Integer counting only, in a fixed order: the permutation is the same on
 // every run.
 //
-// Both passes are chains of latencies.  Few particles (at most kDirectChunks
-// chunks of 512) skip the scan launch: every scattering workgroup sums the
-// few histogram rows itself.  A chunk's keys lie within a few cells of each
-// other, so the ranks come from per-wave counters over a window of the keys
-// (three barriers); a chunk whose keys spread wider takes its waves in turn.
+// Both passes are chains of latencies, so they want many workgroups and few
+// launches: small chunks up to kMidMax particles, and up to kDirectChunks of
+// them without the scan launch (every scattering workgroup sums the histogram
+// rows itself) and with the push inside.  A chunk's keys lie within a few
+// cells of each other, so the ranks come from per-wave counters over a window
+// of the keys (three barriers); a chunk whose keys spread wider takes its
+// waves in turn.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -31,20 +33,28 @@
 
 namespace qpad {
 
-// the two chunk shapes: kSortChunk particles by 1024 threads, or 512 by 512
-constexpr int kSortChunk = 2048;
-constexpr int kDirectChunk = 512;
-constexpr int kDirectChunks = 32;
-constexpr int kDirectBins = 4097;     // bins the direct form keeps in LDS
+// the forms, by the number of particles (sort_args):
+//   direct  chunks of kSmallChunk, no scan launch, the push in the passes;
+//   mid     chunks of kMidChunk;
+//   large   chunks of kSortChunk (fewer histogram rows).
+enum { SORT_LARGE = 0, SORT_MID = 1, SORT_DIRECT = 2, SORT_FORMS = 3 };
+constexpr int kSortChunk = 2048, kSortThreads = 1024;
+constexpr int kMidChunk = 1024, kMidThreads = 512;
+constexpr int kSmallChunk = 512;             // and threads
+constexpr int64_t kMidMax = 131072;          // most particles of the mid form
+constexpr int kDirectChunks = 120;           // most chunks of the direct form
+constexpr int64_t kDirectWork = 1 << 17;     // most (chunks x bins) it sums in every workgroup
+constexpr int kDirectBins = 4097;            // bins the direct form keeps in LDS
+static_assert(kDirectChunks * kSmallChunk < 65536, "the direct form counts in 16 bits");
 
 struct SortArgs {
     int64_t n;
     int nb;                 // bins: keys 0 .. nb-1
     int nchunks;
-    int direct;             // 1: chunks of kDirectChunk, no scan launch
+    int form;               // SORT_*
     const uint32_t *key;
     uint32_t *key_w;        // counting pass of the push: keys out
-    int *hist;              // [nchunks][nb]
+    int *hist;              // [nchunks][nb]; direct: 16-bit rows of hist16_row(nb)
     int *tot;               // [nb]
     int32_t *cs;            // [nb + 1]
     const double *s[8];
@@ -55,6 +65,9 @@ struct SortArgs {
     int4 *desc;             // [n_crowd_max] (cell, first particle, end, overflow row or -1)
     int n_ov_max, n_crowd_max, first;
 };
+
+// row length of the direct form's 16-bit histogram rows (16-byte loads)
+__host__ __device__ inline int hist16_row(int nb) { return (nb + 7) & ~7; }
 
 // particle of this thread in round j of the chunk (a wave owns 64 PER
 // consecutive particles)
@@ -68,14 +81,86 @@ __device__ __forceinline__ int64_t sort_element(int j)
 template <int T, int PER>
 __device__ __forceinline__ void chunk_hist(const SortArgs &a, const uint32_t (&kv)[PER], int *cnt)
 {
+    const bool direct = a.form == SORT_DIRECT;
     for (int b = threadIdx.x; b < a.nb; b += T) cnt[b] = 0;
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PER; j++)
         if (sort_element<T, PER>(j) < a.n) atomicAdd(&cnt[min(kv[j], (uint32_t)(a.nb - 1))], 1);
     __syncthreads();
-    int *h = a.hist + (size_t)blockIdx.x * a.nb;
-    for (int b = threadIdx.x; b < a.nb; b += T) h[b] = cnt[b];
+    if (direct) {
+        const int row = hist16_row(a.nb);
+        unsigned short *h = reinterpret_cast<unsigned short *>(a.hist) + (size_t)blockIdx.x * row;
+        for (int b = threadIdx.x; b < row; b += T) h[b] = b < a.nb ? (unsigned short)cnt[b] : (unsigned short)0;
+    } else {
+        int *h = a.hist + (size_t)blockIdx.x * a.nb;
+        for (int b = threadIdx.x; b < a.nb; b += T) h[b] = cnt[b];
+    }
+}
+
+// direct form: total of every bin into base, the counts of the chunks before
+// this workgroup's into off.  8 bins (16 bytes) a thread, the chunks shared by
+// groups of threads, their rows loaded 8 at a time; the counts stay below
+// 65536 and are added in pairs
+template <int T>
+__device__ __forceinline__ void sum_rows(const SortArgs &a, int *base, int *off)
+{
+    constexpr int R = 8;
+    const int t = threadIdx.x, own = min((int)blockIdx.x, a.nchunks), row = hist16_row(a.nb), nv = row / 8;
+    if (a.nchunks <= R) {
+        // one round of loads without groups
+        const uint32_t *h = reinterpret_cast<const uint32_t *>(a.hist);
+        for (int v = t; 2 * v < a.nb; v += T) {
+            uint32_t x[R], total = 0, mine = 0;
+#pragma unroll
+            for (int u = 0; u < R; u++) x[u] = h[max(min(u, a.nchunks - 1), 0) * (row / 2) + v];
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                total += u < a.nchunks ? x[u] : 0u;
+                mine += u < own ? x[u] : 0u;
+            }
+            *reinterpret_cast<int2 *>(base + 2 * v) = make_int2((int)(total & 0xffffu), (int)(total >> 16));
+            *reinterpret_cast<int2 *>(off + 2 * v) = make_int2((int)(mine & 0xffffu), (int)(mine >> 16));
+        }
+        return;
+    }
+    const int groups = max(T / nv, 1);
+    for (int q = t; q < a.nb; q += T) {
+        base[q] = 0;
+        off[q] = 0;
+    }
+    __syncthreads();
+    const int grp = groups == 1 ? 0 : t / nv;
+    if (grp >= groups) return;
+    for (int v = t - grp * nv; v < nv; v += T) {
+        const uint4 *h = reinterpret_cast<const uint4 *>(a.hist) + v;
+        uint32_t total[4] = {0, 0, 0, 0}, mine[4] = {0, 0, 0, 0};
+        for (int c0 = grp; c0 < a.nchunks; c0 += R * groups) {
+            uint4 x[R];
+#pragma unroll
+            for (int u = 0; u < R; u++) x[u] = h[min(c0 + u * groups, a.nchunks - 1) * nv];
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                const int c = c0 + u * groups;
+                const uint32_t y[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    total[e] += c < a.nchunks ? y[e] : 0u;
+                    mine[e] += c < own ? y[e] : 0u;
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int q = 8 * v + e;
+            const int tv = (int)((total[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+            const int mv = (int)((mine[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+            if (tv && q < a.nb) {
+                atomicAdd(&base[q], tv);
+                if (mv) atomicAdd(&off[q], mv);
+            }
+        }
+    }
 }
 
 // bin starts into base; with `direct` also this chunk's offset within each
@@ -85,19 +170,8 @@ __device__ inline void bin_starts(const SortArgs &a, int *base, int *off)
 {
     __shared__ int wsum[T / 64];
     const int t = threadIdx.x;
-    if (a.direct) {
-        const int own = min((int)blockIdx.x, a.nchunks);
-        for (int q = t; q < a.nb; q += T) {
-            int total = 0, mine = 0;
-#pragma unroll 8
-            for (int c = 0; c < a.nchunks; c++) {
-                const int v = a.hist[(size_t)c * a.nb + q];
-                mine += c < own ? v : 0;
-                total += v;
-            }
-            base[q] = total;
-            off[q] = mine;
-        }
+    if (a.form == SORT_DIRECT) {
+        sum_rows<T>(a, base, off);
     } else {
         for (int q0 = 0; q0 < a.nb; q0 += 8 * T) {
             int v[8];
@@ -313,9 +387,9 @@ __device__ inline void overflow_chunks(const SortArgs &a, const int *base)
 // dynamic LDS of a scattering workgroup: bin starts, offsets (direct), rank
 // counters
 template <int T>
-inline size_t scatter_lds(int nb, bool direct)
+inline size_t scatter_lds(int nb, int form)
 {
-    return sizeof(int) * (size_t)nb * (direct ? 2 : 1) + sizeof(unsigned short) * (size_t)sort_counters<T>();
+    return sizeof(int) * (size_t)hist16_row(nb) * (form == SORT_DIRECT ? 2 : 1) + sizeof(unsigned short) * (size_t)sort_counters<T>();
 }
 
 // the scattering pass up to the positions: destination of each of this
@@ -324,8 +398,8 @@ inline size_t scatter_lds(int nb, bool direct)
 template <int T, int PER>
 __device__ __forceinline__ bool scatter_positions(const SortArgs &a, const uint32_t (&kv)[PER], int *lds, int (&dp)[PER])
 {
-    int *base = lds, *off = lds + a.nb;
-    unsigned short *cnt = reinterpret_cast<unsigned short *>(lds + (size_t)a.nb * (a.direct ? 2 : 1));
+    int *base = lds, *off = lds + hist16_row(a.nb);
+    unsigned short *cnt = reinterpret_cast<unsigned short *>(lds + (size_t)hist16_row(a.nb) * (a.form == SORT_DIRECT ? 2 : 1));
     bin_starts<T>(a, base, off);
     if ((int)blockIdx.x == a.nchunks) {
         for (int b = threadIdx.x; b < a.nb; b += T) a.cs[b] = base[b];
@@ -335,7 +409,7 @@ __device__ __forceinline__ bool scatter_positions(const SortArgs &a, const uint3
     }
     int rank[PER];
     chunk_ranks<T, PER>(a, kv, cnt, rank);
-    const int *row = a.direct ? off : a.hist + (size_t)blockIdx.x * a.nb;
+    const int *row = a.form == SORT_DIRECT ? off : a.hist + (size_t)blockIdx.x * a.nb;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const bool live = sort_element<T, PER>(j) < a.n && kv[j] < (uint32_t)(a.nb - 1);

@@ -1,10 +1,12 @@
 """The re-sort by radial cell at the sizes where its forms meet: one
-particle, chunk edges of both chunk shapes (512 and 2048), the most particles
-of the form without a scan launch (16384) and one more, cell counts on both
-sides of the rank window and of the bins that form keeps in LDS.  Particles
-handed over in random order spread every chunk over all cells (the ranks taken
-in turn), nearly sorted ones stay within the window; some lie outside the box
-and are removed.  The order is exact: by cell, then by the order given."""
+particle, chunk edges of the three chunk shapes (512, 1024 and 2048), the most
+chunks whose rows one round of loads sums (8), the most particles of the form
+without a scan launch (120 chunks of 512, and 131072 chunk counts) and one
+more, the most of the mid form (131072), cell counts on both sides of the rank
+window and of the bins the direct form keeps in LDS.  Particles handed over in
+random order spread every chunk over all cells (the ranks taken in turn),
+nearly sorted ones stay within the window; some lie outside the box and are
+removed.  The order is exact: by cell, then by the order given."""
 import numpy as np
 import pytest
 
@@ -19,7 +21,8 @@ def _ppc(n, nr):
 
 
 @pytest.mark.parametrize("nr,n", [(40, 1), (40, 511), (40, 513), (600, 4096), (1100, 16384), (1100, 16385),
-                                  (2100, 2049), (4200, 9000), (4200, 70001)])
+                                  (2100, 2049), (4200, 9000), (4200, 70001), (40, 4097), (256, 12288), (1000, 61440),
+                                  (1000, 61441), (2100, 31744), (2100, 31745), (600, 131072), (600, 131073)])
 @pytest.mark.parametrize("spread", [False, True])
 def test_sort_is_stable_and_complete(nr, n, spread):
     sim = Simulation(configs.small(nr=nr, nxi=2, max_mode=0, ppc=_ppc(n, nr), total_num=16))
@@ -44,12 +47,12 @@ def test_sort_is_stable_and_complete(nr, n, spread):
     sim.close()
 
 
-@pytest.mark.parametrize("ppc,direct", [((2, 16), True), ((4, 130), False)])
+@pytest.mark.parametrize("ppc,direct", [((2, 16), True), ((4, 130), True), ((4, 260), False)])
 def test_push_forms_keep_the_sorted_order(ppc, direct):
     """both push forms leave the particles grouped by cell, each cell in the
     order its particles had before (no particle lost or doubled)"""
     sim = Simulation(configs.small(nr=64, nxi=40, max_mode=1, ppc=ppc, total_num=1 << 12, offset_x=0.02))
-    assert (64 * ppc[0] * ppc[1] <= 16384) == direct
+    assert (64 * ppc[0] * ppc[1] <= 120 * 512) == direct
     sim.step3d_begin()
     n0 = sim.spe[0].count()
     for j in range(1, 31):
