@@ -121,20 +121,15 @@ __device__ __forceinline__ void wave_reduce_scatter(double (&acc)[16 * NB])
     wave_reduce_from<NB, 0>(acc);
 }
 
-// Level-L value i of values generated on the fly: t0(v), v < 16 NB, is a
-// lane's level-0 value v.  Only the values feeding value i are live, so a
-// lane can add a pass's contributions into level-L accumulators without
-// holding all 16 NB of them.
-template <int NB, int L, class T0>
-__device__ __forceinline__ double reduced_value(const T0 &t0, int i, int lane)
+// 64-lane sum of v in every lane, in a fixed order
+__device__ __forceinline__ double wave_sum(double v)
 {
-    if constexpr (L == 0) {
-        return t0(i);
-    } else {
-        constexpr int half = (8 * NB) >> (L - 1);
-        return reduce_pair<L - 1>(reduced_value<NB, L - 1>(t0, i, lane),
-                                  reduced_value<NB, L - 1>(t0, half + i, lane), lane);
-    }
+    v += dpp<kDppQuadXor1>(v);
+    v += dpp<kDppQuadXor2>(v);
+    v += dpp<kDppRowHalfMirror>(v);
+    v += dpp<kDppRowMirror>(v);
+    v = swap16_sum(v, v);
+    return swap32_sum(v, v);
 }
 
 }  // namespace qpad
