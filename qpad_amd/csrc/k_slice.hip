@@ -783,6 +783,12 @@ __global__ __launch_bounds__(kNodeThreads) void k_start_src(StartSrcArgs a)
         d1[s] = a.P1[s][c1];
         qb[s] = a.qn[s] ? a.qn[s][(size_t)k * ld + i] : 0.0;
     }
+    // the sources' J predictor is requested with the partials, before the
+    // first store (which the compiler must assume to alias it)
+    const int ic = min(max(i, 1), nr);
+    const FieldArr cu{a.cu, nm, ld};
+    const double bz = bz_source(g, cu, k, ic);
+    const double ez = (m == 0) ? ez_source_0(g, cu, ic) : ez_source_m(g, cu, k, ic);
     if (ovf) {
         // overflow rows of crowded cells, in row order (cell_partial)
 #pragma unroll
@@ -805,10 +811,9 @@ __global__ __launch_bounds__(kNodeThreads) void k_start_src(StartSrcArgs a)
         if (a.qn[s]) v = v + qb[s];
     a.q_spe[(size_t)k * ld + i] = v;
     if (i < 1 || i > nr) return;
-    const FieldArr cu{a.cu, nm, ld};
     a.src[(size_t)src_psi(M, nm, k) * nr + i - 1] = -1.0 * v;
-    a.src[(size_t)src_bz(M, k) * nr + i - 1] = bz_source(g, cu, k, i);
-    a.src[(size_t)src_ez(M, nm, k) * nr + i - 1] = (m == 0) ? ez_source_0(g, cu, i) : ez_source_m(g, cu, k, i);
+    a.src[(size_t)src_bz(M, k) * nr + i - 1] = bz;
+    a.src[(size_t)src_ez(M, nm, k) * nr + i - 1] = ez;
 }
 
 struct StartSolveArgs {
@@ -876,55 +881,71 @@ struct EperpArgs {
 
 // thread per (node i = 0..nr+1, mode array k): the iteration's seed into
 // b_spe (when given), b = b_spe + b_beam and E_perp from b and psi
-// (field_e_class.f03:443-504); the k = 0 threads also run 'record' of
-// sum_m |B_phi,m| at their node (simulation_class.f03:549-558) and reset
-// the iteration state.  The first kernel of the slice that reads B_perp.
+// (field_e_class.f03:443-504); one more row of workgroups (k = nm) runs
+// 'record' of sum_m |B_phi,m| (simulation_class.f03:549-558) and resets the
+// iteration state.  The first kernel of the slice that reads B_perp.  A chain
+// of latencies: every load is issued before the first store, and 'record' has
+// threads of its own (MI355X, mean launch, loads between the stores and
+// 'record' by the k = 0 threads before: 256 nodes, M = 1 4.2 -> 3.5 us; 512, M = 0
+// 3.8 -> 3.0; 2048, M = 4 6.5 -> 4.6; 4096, M = 2 5.7 -> 4.5)
+template <int M>
 __global__ __launch_bounds__(kNodeThreads) void k_eperp(EperpArgs a)
 {
+    constexpr int NM = 2 * M + 1;
     const FieldCommon &g = a.g;
-    const int nm = g.nm, ld = g.ld, nr = g.nr, M = g.M;
+    const int nm = NM, ld = g.ld, nr = g.nr;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int k = blockIdx.y;
     if (i > nr + 1) return;
     const bool inner = i >= 1 && i <= nr;
     // B_perp of the iteration's start: the seed, or b_spe as it is
     const double *bperp = (a.seed && inner) ? a.seed : a.b_spe;
-    if (k == 0) {
+    if (k == NM) {
         if (i == 0) {
             a.it->done = 0;
             a.it->iters = 0;
             a.it->counter = 0;
         }
-        if (inner) {
-            double re = 0.0, im = 0.0;
-            for (int mm = 0; mm <= M; mm++) {
-                re = re + fabs(FX(bperp, 1, kre(mm), i));
-                if (mm > 0) im = im + fabs(FX(bperp, 1, kim(mm), i));
-            }
-            a.conv_re[i] = re;
-            a.conv_im[i] = im;
+        if (!inner) return;
+        double v[NM], re = 0.0, im = 0.0;
+#pragma unroll
+        for (int q = 0; q < NM; q++) v[q] = FX(bperp, 1, q, i);
+#pragma unroll
+        for (int mm = 0; mm <= M; mm++) {
+            re = re + fabs(v[mm == 0 ? 0 : 2 * mm - 1]);
+            if (mm > 0) im = im + fabs(v[2 * mm]);
         }
+        a.conv_re[i] = re;
+        a.conv_im[i] = im;
+        return;
     }
-    double bv[3];
+    double bs[3], bb[3], pw[4];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        const double bs = FX(c < 2 ? bperp : a.b_spe, c, k, i);
-        if (c < 2 && a.seed && inner) FX(a.b_spe, c, k, i) = bs;
-        bv[c] = bs + FX(a.b_beam, c, k, i);
+        bs[c] = FX(c < 2 ? bperp : a.b_spe, c, k, i);
+        bb[c] = FX(a.b_beam, c, k, i);
+    }
+    const double ez = FX(a.e, 2, k, i), e0 = FX(a.e, 0, k, i), e1 = FX(a.e, 1, k, i);
+    const double *psik = a.psi + (size_t)k * ld, *psip = a.psi + (size_t)partner(k) * ld;
+#pragma unroll
+    for (int w = 0; w < 4; w++) pw[w] = psik[min(max(i - 2 + w, 0), nr + 1)];
+    const double pp_i = psip[i], pp_2 = psip[2];
+    double bv[3], ev[2] = {e0, e1};
+#pragma unroll
+    for (int c = 0; c < 3; c++) bv[c] = bs[c] + bb[c];
+    if (inner) et_window(g, bv[0], bv[1], pw[0], pw[1], pw[2], pw[3], pp_i, pp_2, k, i, ev);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        if (c < 2 && a.seed && inner) FX(a.b_spe, c, k, i) = bs[c];
         FX(a.b_out, c, k, i) = bv[c];
     }
-    double ev[2];
     if (inner) {
-        et_node(g, bv[0], bv[1], FieldArr{a.psi, nm, ld}, k, i, ev);
         FX(a.e, 0, k, i) = ev[0];
         FX(a.e, 1, k, i) = ev[1];
-    } else {
-        ev[0] = FX(a.e, 0, k, i);
-        ev[1] = FX(a.e, 1, k, i);
     }
     double2 *eb = reinterpret_cast<double2 *>(a.eb + ((size_t)i * nm + k) * 6);
     eb[0] = make_double2(ev[0], ev[1]);
-    eb[1] = make_double2(FX(a.e, 2, k, i), bv[0]);
+    eb[1] = make_double2(ez, bv[0]);
     eb[2] = make_double2(bv[1], bv[2]);
 }
 
@@ -1005,7 +1026,7 @@ int launch_start_solves(qpad_ctx *c)
 int launch_start_eperp(qpad_ctx *c, int j, const double *seed)
 {
     const int nm = c->g.nm;
-    const dim3 ngrid((unsigned)node_blocks(c->g.nr), nm);
+    const dim3 ngrid((unsigned)node_blocks(c->g.nr), nm + 1);
     EperpArgs e;
     e.g = field_common(c);
     e.b_spe = c->f[QPAD_F_B_SPE];
@@ -1018,7 +1039,13 @@ int launch_start_eperp(qpad_ctx *c, int j, const double *seed)
     e.conv_re = c->conv_re;
     e.conv_im = c->conv_im;
     e.it = c->it;
-    hipLaunchKernelGGL(k_eperp, ngrid, dim3(kNodeThreads), 0, c->stream, e);
+    switch (c->g.M) {
+    case 0: hipLaunchKernelGGL(k_eperp<0>, ngrid, dim3(kNodeThreads), 0, c->stream, e); break;
+    case 1: hipLaunchKernelGGL(k_eperp<1>, ngrid, dim3(kNodeThreads), 0, c->stream, e); break;
+    case 2: hipLaunchKernelGGL(k_eperp<2>, ngrid, dim3(kNodeThreads), 0, c->stream, e); break;
+    case 3: hipLaunchKernelGGL(k_eperp<3>, ngrid, dim3(kNodeThreads), 0, c->stream, e); break;
+    default: hipLaunchKernelGGL(k_eperp<4>, ngrid, dim3(kNodeThreads), 0, c->stream, e); break;
+    }
     QPAD_HIP_CHECK(hipGetLastError());
     return 0;
 }
