@@ -1619,7 +1619,7 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form)
         if (form == SORT_DIRECT) {                                                                                    \
             if (maxc) hipLaunchKernelGGL((k_push_keys<MM, STD, PGC>), cg, blk, clds, c->stream, m);       \
             hipLaunchKernelGGL((k_push_scatter<MM, STD, PGC>), mg, blk, mlds, c->stream, m);              \
-        } else {                                                                                         \
+        } else if (nmax) {                                                                               \
             hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(256), 0, c->stream, m);                   \
         }                                                                                                \
     } while (0)

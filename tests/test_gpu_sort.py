@@ -63,3 +63,12 @@ def test_push_forms_keep_the_sorted_order(ppc, direct):
     assert len(np.unique(p["id"])) == len(p["id"]) <= n0
     assert np.all(np.isfinite(p["gamma"])) and np.max(np.abs(p["p1"])) > 1e-3
     sim.close()
+
+
+def test_species_without_particles_on_a_large_grid():
+    """a gas that has released nothing yet, on a grid past the direct form's
+    bins: its push and sort launch for no particles"""
+    sim = Simulation(configs.ionization(nr=4200, nxi=6, max_mode=0, total_num=1 << 10, n_peak=1e-3))
+    sim.step3d()
+    assert sim.neut[0].count() == 0
+    sim.close()
