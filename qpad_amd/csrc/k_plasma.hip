@@ -16,6 +16,7 @@
 
 #include "kernels.h"
 #include "sort_config.h"
+#include "epilogue.h"
 #include "sort_device.h"
 #include "rng.h"
 #include "wave_reduce.h"
@@ -1371,9 +1372,13 @@ struct PushArgs {
     SortArgs s;
 };
 
+constexpr int kPushThreads = 256;
+
 // the arguments of every species of one launch (workgroup rows by species)
 struct PushMulti {
     PushArgs s[kMaxSpecies];
+    int n;       // species; workgroup row n is the slice's epilogue
+    EpiArgs epi;
 };
 
 // STD: push_u_std_part2d (part2d_class.f03:1790-1877), normalised by the
@@ -1508,6 +1513,10 @@ struct Loaded {
 template <int M, bool STD, bool PGC>
 __global__ __launch_bounds__(kSmallChunk) void k_push_keys(const PushMulti m)
 {
+    if ((int)blockIdx.y == m.n) {
+        epilogue_block<kSmallChunk>(m.epi, blockIdx.x);
+        return;
+    }
     const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     if ((int)blockIdx.x >= a.s.nchunks) return;
     extern __shared__ __attribute__((aligned(16))) int lds[];
@@ -1549,8 +1558,12 @@ __global__ __launch_bounds__(kSmallChunk) void k_push_scatter(const PushMulti m)
 }
 
 template <int M, bool STD, bool PGC>
-__global__ __launch_bounds__(256) void k_push(const PushMulti m)
+__global__ __launch_bounds__(kPushThreads) void k_push(const PushMulti m)
 {
+    if ((int)blockIdx.y == m.n) {
+        epilogue_block<kPushThreads>(m.epi, blockIdx.x);
+        return;
+    }
     const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= a.s.n) return;
@@ -1595,7 +1608,7 @@ static PushArgs push_args(qpad_ctx *c, int s)
 // the species of list entries (all of the push type STD, PGC names and all
 // in one sort form)
 template <bool STD, bool PGC>
-static int launch_move_list(qpad_ctx *c, const int *list, int n, int form)
+static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &epi)
 {
     PushMulti m;
     SortMulti sm;
@@ -1610,7 +1623,18 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form)
         nmax = std::max(nmax, m.s[i].s.n);
     }
     const int nb = c->g.nr + 1;
-    const dim3 cg(maxc, n), mg(maxc + 1, n), blk(kSmallChunk), pg((unsigned)((nmax + 255) / 256), n);
+    // the slice's epilogue (epi > 0) rides with the first launch that moves
+    // particles
+    unsigned rows = n, eb = 0;
+    m.n = n;
+    if (epi > 0 && nmax > 0) {
+        m.epi = epilogue_args(c, epi);
+        eb = (unsigned)(epilogue_row_blocks(c->g.nr, form == SORT_DIRECT ? kSmallChunk : kPushThreads) * c->g.nm);
+        rows = n + 1;
+        epi = 0;
+    }
+    const dim3 cg(std::max((unsigned)maxc, eb), rows), mg(maxc + 1, n), blk(kSmallChunk);
+    const dim3 pg(std::max((unsigned)((nmax + kPushThreads - 1) / kPushThreads), eb), rows);
     const size_t clds = sizeof(int) * (size_t)nb, mlds = scatter_lds<kSmallChunk>(nb, SORT_DIRECT);
     hipEvent_t stop = nullptr;
     time_begin(c, 1, &stop);
@@ -1620,7 +1644,7 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form)
             if (maxc) hipLaunchKernelGGL((k_push_keys<MM, STD, PGC>), cg, blk, clds, c->stream, m);       \
             hipLaunchKernelGGL((k_push_scatter<MM, STD, PGC>), mg, blk, mlds, c->stream, m);              \
         } else if (nmax) {                                                                               \
-            hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(256), 0, c->stream, m);                   \
+            hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(kPushThreads), 0, c->stream, m);                   \
         }                                                                                                \
     } while (0)
     switch (c->g.M) {
@@ -1639,8 +1663,8 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form)
 }
 
 // species s0 .. s1-1: one set of launches per push (the two PGC pushers push
-// alike) and sort form present
-static int launch_move_range(qpad_ctx *c, int s0, int s1)
+// alike) and sort form present, the first with slice epi's epilogue (0: none)
+static int launch_move_range(qpad_ctx *c, int s0, int s1, int epi)
 {
     for (int g = 0; g < 3; g++)
         for (int form = 0; form < SORT_FORMS; form++) {
@@ -1649,16 +1673,16 @@ static int launch_move_range(qpad_ctx *c, int s0, int s1)
                 if (std::min(push_group(c->sp[s].cfg.push_type), 2) == g && sort_args(c, s).form == form)
                     list[n++] = s;
             if (!n) continue;
-            if (g == 0) QPAD_TRY((launch_move_list<false, false>(c, list, n, form)));
-            else if (g == 1) QPAD_TRY((launch_move_list<true, false>(c, list, n, form)));
-            else QPAD_TRY((launch_move_list<false, true>(c, list, n, form)));
+            if (g == 0) QPAD_TRY((launch_move_list<false, false>(c, list, n, form, epi)));
+            else if (g == 1) QPAD_TRY((launch_move_list<true, false>(c, list, n, form, epi)));
+            else QPAD_TRY((launch_move_list<false, true>(c, list, n, form, epi)));
         }
-    return 0;
+    return epi > 0 ? launch_epilogue(c, epi) : 0;   // no particles
 }
 
-int launch_move(qpad_ctx *c, int s) { return launch_move_range(c, s, s + 1); }
+int launch_move(qpad_ctx *c, int s) { return launch_move_range(c, s, s + 1, 0); }
 
-int launch_move_all(qpad_ctx *c) { return launch_move_range(c, 0, c->nspecies); }
+int launch_move_all(qpad_ctx *c, int epi) { return launch_move_range(c, 0, c->nspecies, epi); }
 
 // ---------------------------------------------------------------------------
 // interp_psi_part2d (part2d_class.f03:2264-2305): the field psi at every

@@ -1077,11 +1077,14 @@ static int slice_finish(qpad_ctx *c, SliceRun &st)
         TRY(launch_iter_fold(c, false));
         for (int s = 0; s < c->nspecies; s++)
             if (c->sp[s].neutral) TRY(launch_neutral_update(c, s));
-        TRY(launch_move_all(c));
+        TRY(launch_move_all(c, 0));
         st.sub++;
         return subcycle_start(c, st);
     }
-    TRY(launch_epilogue(c, j));
+    // the epilogue runs within the push launch (one launch of 4-6 us less a
+    // slice) unless the network's work waits for it
+    const bool net = seednet_active(c);
+    if (net) TRY(launch_epilogue(c, j));
     if (c->species_q)
         for (int s = 0; s < c->nspecies; s++) TRY(launch_species_cbq(c, s, j));
     // sim_lasers%deposit_chi (simulation_class.f03:400-401): the particles'
@@ -1097,9 +1100,8 @@ static int slice_finish(qpad_ctx *c, SliceRun &st)
         TRY(launch_copy(c, sp.h_rho + (size_t)j * n1, sp.qn, n1));
         TRY(launch_neutral_update(c, s));
     }
-    const bool net = seednet_active(c);
     if (net) TRY(seednet_mark(c));
-    TRY(launch_move_all(c));
+    TRY(launch_move_all(c, net ? 0 : j));
     if (net) TRY(seednet_after_epilogue(c, j, (st.overlap && j < c->g.nxi) ? j + 1 : 0, true));
     c->dt2d = c->g.dxi;
     c->clamp2d = 0.0;
