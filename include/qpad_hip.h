@@ -400,7 +400,7 @@ int qpad_iteration_policy(qpad_ctx *ctx, int32_t adaptive, int32_t margin);
    dep_cells = radial cells, one wave each, per workgroup of the current and
    charge deposits (2, 4 or 8; default 4; results do not depend on it);
    dep_mfma = 1: the current deposit sums each cell's particles on the matrix
-   cores (FP64 MFMA), 0: with the wave reduce-scatter; the two forms add the
+   cores (FP64 MFMA), 0: in lane accumulators; the two forms add the
    same terms in different orders (results equal to rounding), so the form
    is chosen here and never by the autotuner (default: 1 for max_mode >= 3,
    where it measured faster on MI355X, else 0). */
@@ -449,7 +449,7 @@ int qpad_set_beam(qpad_ctx *ctx, int32_t ib, int64_t n, const double *x1,
    sampled on the first predictor-corrector iteration of every slice (which
    always does work; events around every launch would slow the step):
    which = 0: plasma current deposit (amjdeposit), 1: plasma push (every
-   slice), 2: the field sources and solves of the first iteration.  Returns
+   slice; with the re-sort where that runs inside it), 2: the field sources and solves of the first iteration.  Returns
    the summed milliseconds and the number of timed launches since the last
    reset. */
 int qpad_kernel_time(qpad_ctx *ctx, int32_t which, double *ms, int64_t *launches);

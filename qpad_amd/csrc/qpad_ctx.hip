@@ -470,8 +470,9 @@ int qpad_create(const qpad_grid *gr, qpad_ctx **out)
     c->last_dsub = g.dxi;
     c->dep_cells = kDepWaves;
     // the matrix form where it measured faster on MI355X: modes 0..3 and up
-    // (C3, modes 0..4: 18.6 against 26.0 us per current deposit); the
-    // reduce-scatter up to modes 0..2 (C2: 21.5 against 27.5 us)
+    // (modes 0..4, 2 x 131,072 particles: 18.2 against 18.4 us per current
+    // deposit); lane accumulators up to modes 0..2 (524,288 particles: 20.0
+    // against 27.5 us)
     c->dep_mfma = gr->max_mode >= 3 ? 1 : 0;
     if (rc) {
         qpad_destroy(c);

@@ -490,7 +490,7 @@ class Simulation:
 
     def deposit_form(self, mfma=None):
         """Get (or set) the current deposit's accumulation form: True = FP64
-        matrix cores, False = wave reduce-scatter (include/qpad_hip.h)."""
+        matrix cores, False = lane accumulators (include/qpad_hip.h)."""
         sh = L.LaunchShape()
         L.check(self.lib.qpad_get_launch_shape(self.ctx, C.byref(sh)))
         if mfma is not None:
