@@ -579,12 +579,6 @@ __device__ __forceinline__ void gather_n(const F &f, double w0, double w1, doubl
     }
 }
 
-template <int M, class F>
-__device__ __forceinline__ void gather3(const F &f, double w0, double w1, double pc, double ps, double out[3])
-{
-    gather_n<M, 3>(f, w0, w1, pc, ps, out);
-}
-
 // E and B at a particle from the packed fields eb[node][k][e_r, e_phi, e_z,
 // b_r, b_phi, b_z] (qpad_ctx::eb), p at node ix: the six sums over (node,
 // mode array) of the field times w_n times the mode's cos or -sin (doubled
@@ -1714,7 +1708,7 @@ __global__ __launch_bounds__(256) void k_interp_psi(const InterpPsiArgs a)
     const int ix = ic + 1;
     const double w1 = pos - (double)ic, w0 = 1.0 - w1;
     // the gather of interp_field (interp_part2d.f03:66-110) for one
-    // component, in gather3's order of operations
+    // component, in gather_n's order of operations
     const double *f = a.f + ix;
     double v = 0.0;
     v = v + f[0] * w0;

@@ -1,19 +1,19 @@
 // k_slice.hip -- the fused B_perp predictor-corrector iteration of a slice
 // (simulation_class.f03:370-398) after the current deposit:
 //
-//   k_src    every node and mode in parallel: cu, acu, amu from the per-cell
-//            deposit partials (written out), dJ/dxi (written out), and the
-//            right-hand sides of every solve of the iteration (B+/B-, Bz,
-//            Ez) into the `src` buffer, rows interleaved for coalescing;
-//   k_solve  one workgroup per system: B_perp (4 systems per mode, then the
-//            recombination, E_perp and b = b_spe + b_beam of that mode), Bz,
-//            Ez; the last B_perp workgroup runs the convergence test.
+//   k_src      every node and mode in parallel: cu, acu, amu from the per-cell
+//              deposit partials (written out), dJ/dxi (written out), and the
+//              right-hand sides of every solve of the iteration (B+/B-, Bz,
+//              Ez) into the `src` buffer, rows interleaved for coalescing;
+//   k_solve    one workgroup per system: B+/B- (4 systems per mode), Bz, Ez;
+//   k_bfields  B_perp from B+/B-, b = b_spe + b_beam, E_perp, E and B packed
+//              per node, the convergence test's maxima.
 //
-// E and b written by k_solve are the fields of the next iteration's deposit
+// E and b written by k_bfields are the fields of the next iteration's deposit
 // (the reference recomputes them at the top of that iteration from the same
-// cu, b_spe and psi).  k_epilogue is the slice's closing copy-out
-// (simulation_class.f03:401-456).  Every kernel returns at once when the
-// device-side `done` flag says the iteration has converged, so iterations
+// cu, b_spe and psi).  The epilogue (epilogue.h) is the slice's closing
+// copy-out (simulation_class.f03:401-456).  Every kernel returns at once when
+// the device-side `done` flag says the iteration has converged, so iterations
 // are enqueued speculatively with no host round trip.
 #include <algorithm>
 #include <cstring>
