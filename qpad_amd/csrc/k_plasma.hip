@@ -26,16 +26,19 @@ namespace qpad {
 
 #define FX(p, c, k, i) (p)[((size_t)(c) * nm + (size_t)(k)) * ld + (size_t)(i)]
 
-// Radius and normalised position without contraction, so that every kernel
-// computes the same cell for the same particle.
+// Radius of a deposit or a gather, contracted as the compiler likes: an ulp
+// between kernels is harmless there (the cell comes from the sort or is
+// clamped, the weights are linear in the position).
 __device__ inline double radius(double x1, double x2)
 {
     return sqrt(__dadd_rn(__dmul_rn(x1, x1), __dmul_rn(x2, x2)));
 }
 
+// The cell of a stored position.  The fma is written out, so that every
+// kernel that asks computes the same cell for the same particle.
 __device__ inline uint32_t cell_key(double x1, double x2, double idr, double edge, int nr)
 {
-    double r = radius(x1, x2);
+    double r = sqrt(fma(x1, x1, x2 * x2));
     if (!(r < edge)) return (uint32_t)nr;   // leaves the box (update_bound)
     int c = (int)__dmul_rn(r, idr);
     return (uint32_t)(c < nr ? c : nr - 1);
@@ -1345,16 +1348,16 @@ int launch_amjdeposit_all(qpad_ctx *c, int l, bool store_diag, bool timed, bool 
 // push_u_robust (part2d_class.f03:1879-1965) + push_x (:2221-2262) + the
 // re-sort by the new cells (update_bound :2307-2353 is the key nr).
 // Particles that already left the box (past cell_start[nr]) keep key nr.
-// Two forms, by the form of the sort (sort_args):
-// - few particles: two launches.  The counting pass pushes them only for
-//   their new cells, the scattering pass pushes them again on the way to their
-//   sorted places; the launches' latencies are all that counts (blowout
-//   deck, 4096 particles in 256 cells, MI355X: push + counting + scan +
-//   scatter 5.4 + 2.9 + 2.8 + 13.0 us, now 5.0 + 6.9 us).
-// - many: the push in place, a thread per particle, then the plain sort.
-//   There the second gather costs more than the traffic it saves (4096
-//   cells, 524,288 particles, modes 0..2: 49.9 us in the two-pass form
-//   against 48 us; 2 x 131,072 particles, modes 0..4: 50.6 against 38 us).
+// The push is in place, a thread per particle, and the key is the cell of the
+// position it stores.  Two forms, by the form of the sort (sort_args):
+// - few particles (direct): the push launch also counts its chunk's keys
+//   (k_push_count) and the scattering pass follows, two launches whose
+//   latencies are all that counts.  MI355X, kernel trace, push + re-sort of a
+//   slice: 4096 particles in 256 cells 5.8 + 5.9 us, 21189 in 1009 cells 6.1 +
+//   9.4; with a second push in the scattering pass instead of the stores here
+//   5.1 + 7.1 and 6.0 + 10.5 us.
+// - many: k_push, then the plain sort's passes; the direct form's sum of every
+//   chunk's counts in each workgroup ends there.
 // ---------------------------------------------------------------------------
 struct PushArgs {
     int nr, ld, nm;
@@ -1362,7 +1365,8 @@ struct PushArgs {
     double clamp;        // expansion-factor clamp of a sub-cycled push (0: none)
     const double *eb;    // the packed E and B of the slice
     const double *ar, *ai, *arg, *aig;   // laser envelope and gradients (PGC)
-    double *x1, *x2, *p1, *p2, *p3, *gamma;   // pushed in place (many particles)
+    double *x1, *x2, *p1, *p2, *p3, *gamma;   // pushed in place
+    const double *psi;   // interpolated psi (standard pusher)
     SortArgs s;
 };
 
@@ -1381,17 +1385,12 @@ struct PushMulti {
 // PGC: push_u_robust_pgc_part2d / push_u_std_pgc_part2d (:1967-2219, the
 // same steps): the standard normalisation, the ponderomotive term in E with
 // the stored gamma, and the new gamma with gam_corr extrapolated half a step
-// in xi (the envelope's xi gradient).  in(f): the particle's values in the
-// order of SortArgs::s (x1, x2, p1, p2, p3, q, gamma, psi).
-struct Pushed {
-    double x1, x2, p1, p2, p3, gamma;
-};
-
-template <int M, bool STD, bool PGC, class L>
-__device__ __forceinline__ Pushed push_particle(const PushArgs &a, const L &in)
+// in xi (the envelope's xi gradient).  Returns the new cell.
+template <int M, bool STD, bool PGC>
+__device__ __forceinline__ uint32_t push_particle(const PushArgs &a, int64_t p)
 {
     const int nm = a.nm, ld = a.ld;
-    double x1 = in(0), x2 = in(1);
+    double x1 = a.x1[p], x2 = a.x2[p];
     double r = radius(x1, x2);
     const double pc = x1 / r, ps = x2 / r;
     double pos = __dmul_rn(r, a.idr);
@@ -1419,7 +1418,7 @@ __device__ __forceinline__ Pushed push_particle(const PushArgs &a, const L &in)
         la.apig[0] = t;
         const double qbm2_hf = a.qbm * a.qbm * 0.5;
         gam_corr = qbm2_hf * (la.apr * la.apr + la.api * la.api);
-        const double tmp = 0.5 * a.qbm / in(6);
+        const double tmp = 0.5 * a.qbm / a.gamma[p];
         ep[0] = ep[0] - tmp * (la.apr * la.aprg[0] + la.api * la.apig[0]);
         ep[1] = ep[1] - tmp * (la.apr * la.aprg[1] + la.api * la.apig[1]);
         ep[2] = ep[2] + tmp * (la.apr * la.aprg[2] + la.api * la.apig[2]);
@@ -1428,11 +1427,11 @@ __device__ __forceinline__ Pushed push_particle(const PushArgs &a, const L &in)
         apr_z = la.aprg[2];
         api_z = la.apig[2];
     }
-    double pp[3] = {in(2), in(3), in(4)}, ut[3];
+    double pp[3] = {a.p1[p], a.p2[p], a.p3[p]}, ut[3];
     double qtmh1, qtmh2;
     if constexpr (STD || PGC) {
-        qtmh1 = a.qtmh / (1.0 - a.qbm * in(7));
-        qtmh2 = qtmh1 * in(6);
+        qtmh1 = a.qtmh / (1.0 - a.qbm * a.psi[p]);
+        qtmh2 = qtmh1 * a.gamma[p];
     } else {
         const double gam = sqrt(1.0 + pp[0] * pp[0] + pp[1] * pp[1] + pp[2] * pp[2]);
         qtmh1 = a.qtmh / (gam - pp[2]);
@@ -1483,29 +1482,19 @@ __device__ __forceinline__ Pushed push_particle(const PushArgs &a, const L &in)
     double dtc = a.dt / (g2 - pp[2]);
     x1 = x1 + pp[0] * dtc;
     x2 = x2 + pp[1] * dtc;
-    Pushed o;
-    o.x1 = x1;
-    o.x2 = x2;
-    o.p1 = pp[0];
-    o.p2 = pp[1];
-    o.p3 = pp[2];
-    o.gamma = g2;
-    return o;
+    a.p1[p] = pp[0];
+    a.p2[p] = pp[1];
+    a.p3[p] = pp[2];
+    a.gamma[p] = g2;
+    a.x1[p] = x1;
+    a.x2[p] = x2;
+    const uint32_t key = cell_key(x1, x2, a.idr, a.edge, a.nr);
+    a.s.key_w[p] = key;
+    return key;
 }
 
-// a particle's values where the pusher asks for them, and loaded beforehand
-struct LoadAt {
-    const SortArgs &s;
-    int64_t p;
-    __device__ __forceinline__ double operator()(int f) const { return s.s[f][p]; }
-};
-struct Loaded {
-    double v[8];
-    __device__ __forceinline__ double operator()(int f) const { return v[f]; }
-};
-
 template <int M, bool STD, bool PGC>
-__global__ __launch_bounds__(kSmallChunk) void k_push_keys(const PushMulti m)
+__global__ __launch_bounds__(kSmallChunk) void k_push_count(const PushMulti m)
 {
     if ((int)blockIdx.y == m.n) {
         epilogue_block<kSmallChunk>(m.epi, blockIdx.x);
@@ -1514,41 +1503,13 @@ __global__ __launch_bounds__(kSmallChunk) void k_push_keys(const PushMulti m)
     const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     if ((int)blockIdx.x >= a.s.nchunks) return;
     extern __shared__ __attribute__((aligned(16))) int lds[];
-    const int live = a.s.cs[a.nr];
     const int64_t p = sort_element<kSmallChunk, 1>(0);
-    const Pushed o = push_particle<M, STD, PGC>(a, LoadAt{a.s, min(p, a.s.n - 1)});
-    const uint32_t kv[1] = {p < live ? cell_key(o.x1, o.x2, a.idr, a.edge, a.nr) : (uint32_t)a.nr};
-    if (p < a.s.n) a.s.key_w[p] = kv[0];
+    uint32_t kv[1] = {(uint32_t)a.nr};
+    if (p < a.s.n) {
+        if (p < a.s.cs[a.nr]) kv[0] = push_particle<M, STD, PGC>(a, p);
+        else a.s.key_w[p] = (uint32_t)a.nr;
+    }
     chunk_hist<kSmallChunk, 1>(a.s, kv, lds);
-}
-
-template <int M, bool STD, bool PGC>
-__global__ __launch_bounds__(kSmallChunk) void k_push_scatter(const PushMulti m)
-{
-    const PushArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
-    if ((int)blockIdx.x > a.s.nchunks) return;
-    extern __shared__ __attribute__((aligned(16))) int lds[];
-    // the particle's loads are issued before the counting, which hides them
-    const int64_t e = max(min(sort_element<kSmallChunk, 1>(0), a.s.n - 1), (int64_t)0);
-    const uint32_t kv[1] = {min(a.s.key[e], (uint32_t)a.nr)};
-    Loaded in;
-#pragma unroll
-    for (int f = 0; f < 8; f++) in.v[f] = a.s.s[f][e];
-    const int32_t id = a.s.sid[e];
-    int dp[1];
-    if (!scatter_positions<kSmallChunk, 1>(a.s, kv, lds, dp)) return;
-    const int at = dp[0];
-    if (at < 0) return;
-    const Pushed o = push_particle<M, STD, PGC>(a, in);
-    a.s.d[0][at] = o.x1;
-    a.s.d[1][at] = o.x2;
-    a.s.d[2][at] = o.p1;
-    a.s.d[3][at] = o.p2;
-    a.s.d[4][at] = o.p3;
-    a.s.d[5][at] = in.v[5];
-    a.s.d[6][at] = o.gamma;
-    a.s.d[7][at] = in.v[7];
-    a.s.did[at] = id;
 }
 
 template <int M, bool STD, bool PGC>
@@ -1566,14 +1527,7 @@ __global__ __launch_bounds__(kPushThreads) void k_push(const PushMulti m)
         a.s.key_w[p] = (uint32_t)a.nr;
         return;
     }
-    const Pushed o = push_particle<M, STD, PGC>(a, LoadAt{a.s, p});
-    a.p1[p] = o.p1;
-    a.p2[p] = o.p2;
-    a.p3[p] = o.p3;
-    a.gamma[p] = o.gamma;
-    a.x1[p] = o.x1;
-    a.x2[p] = o.x2;
-    a.s.key_w[p] = cell_key(o.x1, o.x2, a.idr, a.edge, a.nr);
+    push_particle<M, STD, PGC>(a, p);
 }
 
 static PushArgs push_args(qpad_ctx *c, int s)
@@ -1595,6 +1549,7 @@ static PushArgs push_args(qpad_ctx *c, int s)
     a.arg = c->f[QPAD_F_AR_GRAD];
     a.aig = c->f[QPAD_F_AI_GRAD];
     a.x1 = sp.x1; a.x2 = sp.x2; a.p1 = sp.p1; a.p2 = sp.p2; a.p3 = sp.p3; a.gamma = sp.gamma;
+    a.psi = sp.psi;
     a.s = sort_args(c, s);
     return a;
 }
@@ -1627,19 +1582,16 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &
         rows = n + 1;
         epi = 0;
     }
-    const dim3 cg(std::max((unsigned)maxc, eb), rows), mg(maxc + 1, n), blk(kSmallChunk);
+    const dim3 cg(std::max((unsigned)maxc, eb), rows), blk(kSmallChunk);
     const dim3 pg(std::max((unsigned)((nmax + kPushThreads - 1) / kPushThreads), eb), rows);
-    const size_t clds = sizeof(int) * (size_t)nb, mlds = scatter_lds<kSmallChunk>(nb, SORT_DIRECT);
+    const size_t clds = sizeof(int) * (size_t)nb;
     hipEvent_t stop = nullptr;
     time_begin(c, 1, &stop);
-#define QPAD_MOVE(MM)                                                                                    \
-    do {                                                                                                 \
-        if (form == SORT_DIRECT) {                                                                                    \
-            if (maxc) hipLaunchKernelGGL((k_push_keys<MM, STD, PGC>), cg, blk, clds, c->stream, m);       \
-            hipLaunchKernelGGL((k_push_scatter<MM, STD, PGC>), mg, blk, mlds, c->stream, m);              \
-        } else if (nmax) {                                                                               \
-            hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(kPushThreads), 0, c->stream, m);                   \
-        }                                                                                                \
+#define QPAD_MOVE(MM)                                                                                 \
+    do {                                                                                              \
+        if (!nmax) break;                                                                             \
+        if (form == SORT_DIRECT) hipLaunchKernelGGL((k_push_count<MM, STD, PGC>), cg, blk, clds, c->stream, m); \
+        else hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(kPushThreads), 0, c->stream, m);      \
     } while (0)
     switch (c->g.M) {
     case 0: QPAD_MOVE(0); break;
@@ -1651,7 +1603,7 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &
 #undef QPAD_MOVE
     QPAD_HIP_CHECK(hipGetLastError());
     time_end(c, 1, stop);
-    if (form != SORT_DIRECT) QPAD_TRY(launch_sort_list(c, sm, n));
+    QPAD_TRY(launch_sort_list(c, sm, n, form == SORT_DIRECT));
     for (int i = 0; i < n; i++) sort_swap(c->sp[list[i]]);
     return 0;
 }

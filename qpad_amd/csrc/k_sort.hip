@@ -1,6 +1,6 @@
-// k_sort.hip -- the plain per-slice re-sort of a plasma species by radial
-// cell (after injection or when the caller sets particles) and the host side
-// of the sort; the passes are described in sort_device.h.
+// k_sort.hip -- the re-sort of a plasma species by radial cell (of a slice,
+// after injection, or when the caller sets particles): its launches and its
+// host side; the passes are described in sort_device.h.
 #include <algorithm>
 #include <cstring>
 #include <string>
@@ -137,8 +137,8 @@ SortArgs sort_args(qpad_ctx *c, int s)
     a.n = n;
     a.nb = c->g.nr + 1;
     // push and re-sort, us a slice, chunks of 2048 with the scan launch -> the
-    // form now: direct 4096 particles in 256 cells 24.1 -> 11.8, 21189 in 1009
-    // 23.4 -> 16.0, 24576 in 768 27 -> 19.5 (the sum over the chunks grows with
+    // form now: direct 4096 particles in 256 cells 24.1 -> 11.7, 21189 in 1009
+    // 23.4 -> 15.5, 24576 in 768 27 -> 19.5 (the sum over the chunks grows with
     // chunks x bins: at 131072 its 2 us equal the scan launch); sort alone, mid
     // form: 65536 in 512 cells 20.0 -> 17.1; two species of 131072 in 2048
     // 22.1 -> 22.1, where the chunk counts' traffic meets the gain
@@ -191,7 +191,7 @@ static int launch_sort_scan(qpad_ctx *c, const SortMulti &m, int ns, int maxc)
     return 0;
 }
 
-int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns)
+int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns, bool counted)
 {
     int maxc = 0;
     for (int i = 0; i < ns; i++) maxc = std::max(maxc, m.s[i].nchunks);
@@ -201,7 +201,7 @@ int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns)
     const dim3 cg(std::max(maxc, 1), ns), mg(maxc + 1, ns);
 #define QPAD_SORT(T, PER)                                                                              \
     do {                                                                                              \
-        if (maxc) hipLaunchKernelGGL((k_sort_hist<T, PER>), cg, dim3(T), hl, c->stream, m);            \
+        if (maxc && !counted) hipLaunchKernelGGL((k_sort_hist<T, PER>), cg, dim3(T), hl, c->stream, m);            \
         if (form != SORT_DIRECT) QPAD_TRY(launch_sort_scan(c, m, ns, maxc));                           \
         hipLaunchKernelGGL((k_sort_scatter<T, PER>), mg, dim3(T), scatter_lds<T>(nb, form), c->stream, m); \
     } while (0)
@@ -218,7 +218,7 @@ int launch_sort(qpad_ctx *c, int s)
     SortMulti m;
     memset(&m, 0, sizeof(m));
     m.s[0] = sort_args(c, s);
-    QPAD_TRY(launch_sort_list(c, m, 1));
+    QPAD_TRY(launch_sort_list(c, m, 1, false));
     sort_swap(c->sp[s]);
     return 0;
 }

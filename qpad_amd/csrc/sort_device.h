@@ -1,8 +1,8 @@
 // sort_device.h -- device side of the per-slice re-sort of a plasma species
 // by radial cell (the order QPAD's update_bound leaves,
 // part2d_class.f03:2307-2353, is not kept: particles are regrouped by cell so
-// that one wave deposits one cell), shared by the plain sort (k_sort.hip) and
-// the push that moves few particles to their sorted places (k_plasma.hip).
+// that one wave deposits one cell), shared by the sort (k_sort.hip) and the
+// push that counts the cells of few particles (k_plasma.hip).
 //
 // Stable counting sort over the nr + 1 cell keys (key nr = left the box),
 // chunk of T * PER particles per workgroup of T threads:
@@ -21,7 +21,7 @@
 // Both passes are chains of latencies, so they want many workgroups and few
 // launches: small chunks up to kMidMax particles, and up to kDirectChunks of
 // them without the scan launch (every scattering workgroup sums the histogram
-// rows itself) and with the push inside.  A chunk's keys lie within a few
+// rows itself) and counted by the push.  A chunk's keys lie within a few
 // cells of each other, so the ranks come from per-wave counters over a window
 // of the keys (three barriers); a chunk whose keys spread wider takes its
 // waves in turn.
@@ -34,7 +34,7 @@
 namespace qpad {
 
 // the forms, by the number of particles (sort_args):
-//   direct  chunks of kSmallChunk, no scan launch, the push in the passes;
+//   direct  chunks of kSmallChunk, no scan launch, counted by the push;
 //   mid     chunks of kMidChunk;
 //   large   chunks of kSortChunk (fewer histogram rows).
 enum { SORT_LARGE = 0, SORT_MID = 1, SORT_DIRECT = 2, SORT_FORMS = 3 };
@@ -424,8 +424,8 @@ struct SortMulti {
     SortArgs s[kMaxSpecies];
 };
 // the sort of the species of m.s[0 .. ns-1], all in one form (workgroup rows
-// by species)
-int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns);
+// by species); counted: the push has counted the keys already
+int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns, bool counted);
 // the sorted buffers become the current ones
 void sort_swap(Species &sp);
 
