@@ -18,6 +18,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include "kernels.h"
+#include "sort_device.h"
 #include "wave_reduce.h"
 
 namespace qpad {
@@ -147,14 +148,6 @@ struct AddArgs {
     double *ax1, *ax2, *aq;
 };
 
-__device__ inline uint32_t neutral_key(double x1, double x2, double idr, double edge, int nr)
-{
-    const double r = sqrt(__dadd_rn(__dmul_rn(x1, x1), __dmul_rn(x2, x2)));
-    if (!(r < edge)) return (uint32_t)nr;
-    const int cc = (int)__dmul_rn(r, idr);
-    return (uint32_t)(cc < nr ? cc : nr - 1);
-}
-
 __global__ __launch_bounds__(256) void k_neutral_add(const AddArgs a)
 {
     const int nc = a.nth * a.nr;
@@ -181,7 +174,7 @@ __global__ __launch_bounds__(256) void k_neutral_add(const AddArgs a)
         a.gamma[p] = 1.0;
         a.psi[p] = 0.0;
         a.id[p] = rel + base + i - 1;
-        a.key[p] = neutral_key(x1, x2, a.idr, a.edge, a.nr);
+        a.key[p] = cell_key(x1, x2, a.idr, a.edge, a.nr);
         a.ax1[base + i - 1] = x1;
         a.ax2[base + i - 1] = x2;
         a.aq[base + i - 1] = -qp;

@@ -34,16 +34,6 @@ __device__ inline double radius(double x1, double x2)
     return sqrt(__dadd_rn(__dmul_rn(x1, x1), __dmul_rn(x2, x2)));
 }
 
-// The cell of a stored position.  The fma is written out, so that every
-// kernel that asks computes the same cell for the same particle.
-__device__ inline uint32_t cell_key(double x1, double x2, double idr, double edge, int nr)
-{
-    double r = sqrt(fma(x1, x1, x2 * x2));
-    if (!(r < edge)) return (uint32_t)nr;   // leaves the box (update_bound)
-    int c = (int)__dmul_rn(r, idr);
-    return (uint32_t)(c < nr ? c : nr - 1);
-}
-
 // ---------------------------------------------------------------------------
 // injection: fdist2d_class.f03:289-357 (lattice theta).  A uniform plasma
 // keeps every lattice point; a profiled one (den_perp given) keeps the points

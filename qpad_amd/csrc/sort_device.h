@@ -47,6 +47,16 @@ constexpr int64_t kDirectWork = 1 << 17;     // most (chunks x bins) it sums in 
 constexpr int kDirectBins = 4097;            // bins the direct form keeps in LDS
 static_assert(kDirectChunks * kSmallChunk < 65536, "the direct form counts in 16 bits");
 
+// The cell of a stored position.  The fma is written out, so that every
+// kernel that asks computes the same cell for the same particle.
+__device__ __forceinline__ uint32_t cell_key(double x1, double x2, double idr, double edge, int nr)
+{
+    double r = sqrt(fma(x1, x1, x2 * x2));
+    if (!(r < edge)) return (uint32_t)nr;   // leaves the box (update_bound)
+    int c = (int)__dmul_rn(r, idr);
+    return (uint32_t)(c < nr ? c : nr - 1);
+}
+
 struct SortArgs {
     int64_t n;
     int nb;                 // bins: keys 0 .. nb-1
