@@ -525,6 +525,7 @@ def main():
                           "frac": step_bytes * steps_per_s / 1e9 / HBM_PEAK_GBS},
         "first_iteration_kernel_ms_per_step": {"amjdeposit": dep_ms / args.steps,
                                                "sources_and_solves": sol_ms / args.steps},
+        # of the reported leg; in the plain leg these launches hold the slices' epilogues
         "push_ms_per_step": push_ms / args.steps,
     }
     legs["learned"].close()

@@ -448,10 +448,12 @@ int qpad_set_beam(qpad_ctx *ctx, int32_t ib, int64_t n, const double *x1,
 /* timing of the dominant kernels (HIP events on the context's stream),
    sampled on the first predictor-corrector iteration of every slice (which
    always does work; events around every launch would slow the step):
-   which = 0: plasma current deposit (amjdeposit), 1: plasma push (every
-   slice; with the re-sort where that runs inside it), 2: the field sources and solves of the first iteration.  Returns
-   the summed milliseconds and the number of timed launches since the last
-   reset. */
+   which = 0: plasma current deposit (amjdeposit), 1: the plasma push launches
+   (every slice, every species with particles; the launch also counts the
+   cells for the re-sort where the particles are few, and the slice's first
+   one holds the slice's epilogue unless the learned seed is on), 2: the field
+   sources and solves of the first iteration.  Returns the summed milliseconds
+   and the number of timed launches since the last reset. */
 int qpad_kernel_time(qpad_ctx *ctx, int32_t which, double *ms, int64_t *launches);
 int qpad_kernel_time_reset(qpad_ctx *ctx, int32_t enable);
 

@@ -1575,24 +1575,25 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &
     const dim3 cg(std::max((unsigned)maxc, eb), rows), blk(kSmallChunk);
     const dim3 pg(std::max((unsigned)((nmax + kPushThreads - 1) / kPushThreads), eb), rows);
     const size_t clds = sizeof(int) * (size_t)nb;
-    hipEvent_t stop = nullptr;
-    time_begin(c, 1, &stop);
-#define QPAD_MOVE(MM)                                                                                 \
-    do {                                                                                              \
-        if (!nmax) break;                                                                             \
+    if (nmax > 0) {
+        hipEvent_t stop = nullptr;
+        time_begin(c, 1, &stop);
+#define QPAD_MOVE(MM)                                                                                       \
+    do {                                                                                                    \
         if (form == SORT_DIRECT) hipLaunchKernelGGL((k_push_count<MM, STD, PGC>), cg, blk, clds, c->stream, m); \
-        else hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(kPushThreads), 0, c->stream, m);      \
+        else hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(kPushThreads), 0, c->stream, m);            \
     } while (0)
-    switch (c->g.M) {
-    case 0: QPAD_MOVE(0); break;
-    case 1: QPAD_MOVE(1); break;
-    case 2: QPAD_MOVE(2); break;
-    case 3: QPAD_MOVE(3); break;
-    default: QPAD_MOVE(4); break;
-    }
+        switch (c->g.M) {
+        case 0: QPAD_MOVE(0); break;
+        case 1: QPAD_MOVE(1); break;
+        case 2: QPAD_MOVE(2); break;
+        case 3: QPAD_MOVE(3); break;
+        default: QPAD_MOVE(4); break;
+        }
 #undef QPAD_MOVE
-    QPAD_HIP_CHECK(hipGetLastError());
-    time_end(c, 1, stop);
+        QPAD_HIP_CHECK(hipGetLastError());
+        time_end(c, 1, stop);
+    }
     QPAD_TRY(launch_sort_list(c, sm, n, form == SORT_DIRECT));
     for (int i = 0; i < n; i++) sort_swap(c->sp[list[i]]);
     return 0;
