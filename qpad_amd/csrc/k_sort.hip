@@ -205,9 +205,9 @@ int launch_sort_list(qpad_ctx *c, const SortMulti &m, int ns, bool counted)
         if (form != SORT_DIRECT) QPAD_TRY(launch_sort_scan(c, m, ns, maxc));                           \
         hipLaunchKernelGGL((k_sort_scatter<T, PER>), mg, dim3(T), scatter_lds<T>(nb, form), c->stream, m); \
     } while (0)
-    if (form == SORT_LARGE) QPAD_SORT(kSortThreads, 2);
-    else if (form == SORT_MID) QPAD_SORT(kMidThreads, 2);
-    else QPAD_SORT(kSmallChunk, 1);
+    if (form == SORT_LARGE) QPAD_SORT(kSortThreads, kSortChunk / kSortThreads);
+    else if (form == SORT_MID) QPAD_SORT(kSortThreads, kMidChunk / kSortThreads);
+    else QPAD_SORT(kSortThreads, kSmallChunk / kSortThreads);
 #undef QPAD_SORT
     QPAD_HIP_CHECK(hipGetLastError());
     return 0;

@@ -38,9 +38,14 @@ namespace qpad {
 //   mid     chunks of kMidChunk;
 //   large   chunks of kSortChunk (fewer histogram rows).
 enum { SORT_LARGE = 0, SORT_MID = 1, SORT_DIRECT = 2, SORT_FORMS = 3 };
-constexpr int kSortChunk = 2048, kSortThreads = 1024;
-constexpr int kMidChunk = 1024, kMidThreads = 512;
-constexpr int kSmallChunk = 512;             // and threads
+constexpr int kSortChunk = 2048;
+constexpr int kMidChunk = 1024;
+constexpr int kSmallChunk = 512;
+// threads of every form's workgroups: with 1024 for the large one, two fit a
+// CU and the closing workgroup waits for a second round (scatter, 2^20
+// particles in 8192 cells 41.5 us, with 512 33.6; 524288 in 4096 20.6, 17.5)
+constexpr int kSortThreads = 512;
+static_assert(kSortThreads == kSmallChunk, "the direct form: a thread per particle");
 constexpr int64_t kMidMax = 131072;          // most particles of the mid form
 constexpr int kDirectChunks = 120;           // most chunks of the direct form
 constexpr int64_t kDirectWork = 1 << 17;     // most (chunks x bins) it sums in every workgroup
@@ -220,12 +225,12 @@ __device__ inline void bin_starts(const SortArgs &a, int *base, int *off)
     __syncthreads();
 }
 
-// key window of the per-wave rank counters (bins); with the counters of T /
-// 64 waves at least as large as one 16-bit counter per bin of 8192 cells
+// key window of the per-wave rank counters (bins); the counters of the waves
+// are together at least one 16-bit counter per bin of 8192 cells
+constexpr int kSortWindow = 1024;
 template <int T>
-constexpr int sort_window() { return T >= 1024 ? 512 : 1024; }
-template <int T>
-constexpr int sort_counters() { return (T / 64) * (sort_window<T>() + 1); }
+constexpr int sort_counters() { return (T / 64) * (kSortWindow + 1); }
+static_assert(sort_counters<kSortThreads>() >= 8192, "chunks whose keys spread wide: a counter per cell");
 
 // lanes of the wave with this lane's value (of `bits` bits)
 __device__ __forceinline__ uint64_t match_lanes(uint32_t v, int bits, bool valid)
@@ -244,7 +249,7 @@ __device__ __forceinline__ uint64_t match_lanes(uint32_t v, int bits, bool valid
 template <int T, int PER>
 __device__ inline void chunk_ranks(const SortArgs &a, const uint32_t (&kv)[PER], unsigned short *cnt, int (&rank)[PER])
 {
-    constexpr int NW = T / 64, W = sort_window<T>();
+    constexpr int NW = T / 64, W = kSortWindow;
     __shared__ int kmin[NW], kmax[NW];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
