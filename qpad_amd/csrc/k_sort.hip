@@ -136,16 +136,19 @@ SortArgs sort_args(qpad_ctx *c, int s)
     memset(&a, 0, sizeof(a));
     a.n = n;
     a.nb = c->g.nr + 1;
-    // push and re-sort, us a slice, chunks of 2048 with the scan launch -> the
-    // form now: direct 4096 particles in 256 cells 24.1 -> 11.7, 21189 in 1009
-    // 23.4 -> 15.5, 24576 in 768 27 -> 19.5 (the sum over the chunks grows with
-    // chunks x bins: at 131072 its 2 us equal the scan launch); sort alone, mid
-    // form: 65536 in 512 cells 20.0 -> 17.1; two species of 131072 in 2048
-    // 22.1 -> 22.1, where the chunk counts' traffic meets the gain
-    const int64_t small = (n + kSmallChunk - 1) / kSmallChunk;
-    if (n > kMidMax) a.form = SORT_LARGE;
-    else if (a.nb > kDirectBins || small > kDirectChunks || small * a.nb > kDirectWork) a.form = SORT_MID;
-    else a.form = SORT_DIRECT;
+    // direct: push and re-sort, us a slice, chunks of 2048 with the scan launch
+    // -> direct: 4096 particles in 256 cells 24.1 -> 11.7, 21189 in 1009 23.4 ->
+    // 15.5, 24576 in 768 27 -> 19.5 (the sum over the chunks grows with chunks x
+    // bins: at 131072 its 2 us equal the scan launch)
+    // mid: the sort's three launches, us, chunks of 2048 -> 1024: 65536 in 512
+    // cells 18.5 -> 15.4, 262144 in 512 21.7 -> 17.9, in 2048 22.1 -> 19.7, in
+    // 4096 23.8 -> 23.1; 131072 in 8192 24.6 -> 24.7.  Past the line the larger
+    // histogram costs more than the shorter chunks give: 393216 in 512 23.6 ->
+    // 23.6, in 2048 24.2 -> 25.2, in 4096 25.7 -> 28.3; 196608 in 8192 26.0 -> 28.4
+    const int64_t small = (n + kSmallChunk - 1) / kSmallChunk, mid = (n + kMidChunk - 1) / kMidChunk;
+    if (a.nb <= kDirectBins && small <= kDirectChunks && small * a.nb <= kDirectWork) a.form = SORT_DIRECT;
+    else if (n <= kMidMax && mid * c->g.nr <= kMidWork) a.form = SORT_MID;
+    else a.form = SORT_LARGE;
     const int chunk = a.form == SORT_LARGE ? kSortChunk : a.form == SORT_MID ? kMidChunk : kSmallChunk;
     a.nchunks = (int)((n + chunk - 1) / chunk);
     a.key = sp.key;

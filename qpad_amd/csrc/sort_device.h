@@ -46,7 +46,8 @@ constexpr int kSmallChunk = 512;
 // particles in 8192 cells 41.5 us, with 512 33.6; 524288 in 4096 20.6, 17.5)
 constexpr int kSortThreads = 512;
 static_assert(kSortThreads == kSmallChunk, "the direct form: a thread per particle");
-constexpr int64_t kMidMax = 131072;          // most particles of the mid form
+constexpr int64_t kMidMax = 262144;          // most particles of the mid form
+constexpr int64_t kMidWork = 1 << 20;        // most (chunks x cells) of its histogram
 constexpr int kDirectChunks = 120;           // most chunks of the direct form
 constexpr int64_t kDirectWork = 1 << 17;     // most (chunks x bins) it sums in every workgroup
 constexpr int kDirectBins = 4097;            // bins the direct form keeps in LDS

@@ -2,7 +2,8 @@
 particle, chunk edges of the three chunk shapes (512, 1024 and 2048), the most
 chunks whose rows one round of loads sums (8), the most particles of the form
 without a scan launch (120 chunks of 512, and 131072 chunk counts) and one
-more, the most of the mid form (131072), cell counts on both sides of the rank
+more, the most of the mid form (262144, and 2^20 chunk counts: 131072 in 8192
+cells) and one more, 131072 and one more well inside it, cell counts on both sides of the rank
 window and of the bins the direct form keeps in LDS.  Particles handed over in
 random order spread every chunk over all cells (the ranks taken in turn),
 nearly sorted ones stay within the window; some lie outside the box and are
@@ -22,7 +23,8 @@ def _ppc(n, nr):
 
 @pytest.mark.parametrize("nr,n", [(40, 1), (40, 511), (40, 513), (600, 4096), (1100, 16384), (1100, 16385),
                                   (2100, 2049), (4200, 9000), (4200, 70001), (40, 4097), (256, 12288), (1000, 61440),
-                                  (1000, 61441), (2100, 31744), (2100, 31745), (600, 131072), (600, 131073)])
+                                  (1000, 61441), (2100, 31744), (2100, 31745), (600, 131072), (600, 131073),
+                                  (600, 262144), (600, 262145), (8192, 131072), (8192, 131073)])
 @pytest.mark.parametrize("spread", [False, True])
 def test_sort_is_stable_and_complete(nr, n, spread):
     sim = Simulation(configs.small(nr=nr, nxi=2, max_mode=0, ppc=_ppc(n, nr), total_num=16))
