@@ -617,7 +617,25 @@ struct UniformFence {
     __device__ __forceinline__ void operator()(uniform_ptr &p) const { __asm__ volatile("" : "+s"(p)); }
 };
 struct NoFence {
-    __device__ __forceinline__ void operator()(const double *) const {}
+    template <class P>
+    __device__ __forceinline__ void operator()(const P &) const {}
+};
+
+// value l = n 6 NM + 6 k + q of the packed layout, for the node pair at ix of
+// the slice fields e and b themselves: what a single call (species2d%amjdp,
+// species2d%push) gathers, whose e and b come from separate solves.  Packing
+// them first is a launch of its own (a call, MI355X: 4096 particles in 256
+// cells, amjdp 22.8 us packed, 19.1 so, push 25.0 and 21.5; 524,288 in 4096,
+// M = 2, 38.1 and 32.7, 63.1 and 56.1).
+template <int NM>
+struct SplitFields {
+    const double *e, *b;
+    int nm, ld, ix;
+    __device__ __forceinline__ double operator[](int l) const
+    {
+        const int n = l / (6 * NM), k = l / 6 % NM, q = l % 6;
+        return (q < 3 ? e : b)[((size_t)(q % 3) * nm + k) * ld + ix + n];
+    }
 };
 
 // nodes ix, ix + 1 of a slice field in HBM
@@ -670,6 +688,7 @@ struct JDepArgs {
     int store_diag;
     const int32_t *cs;
     const double *eb;   // the packed E and B of the slice (qpad_ctx::eb)
+    const double *e, *b;   // the slice fields (single calls)
     // the laser envelope and its gradients of the slice (PGC pushers)
     const double *ar, *ai, *arg, *aig;
     double *P0, *P1;
@@ -739,8 +758,8 @@ __device__ __forceinline__ double dep_stage_load_pgc(const double *ar, const dou
 // normalises its second half kick by gamma / (gamma - u_z) of the rotated
 // momentum.  eb: the packed fields at the cell's left node; sf: the wave's
 // staged laser values (PGC).
-template <int M, bool STD, bool PGC>
-__device__ __forceinline__ void particle_terms(const JDepArgs &a, uniform_ptr eb, const double *sf, int c, int p,
+template <int M, bool STD, bool PGC, class P, class F>
+__device__ __forceinline__ void particle_terms(const JDepArgs &a, P eb, const F &fence, const double *sf, int c, int p,
                                                bool valid,
                                                double x1, double x2, double pp1, double pp2, double pp3, double qp,
                                                double psip, PartTerms<M> &t)
@@ -751,7 +770,7 @@ __device__ __forceinline__ void particle_terms(const JDepArgs &a, uniform_ptr eb
     double pos = __dmul_rn(r, a.idr);
     const double w1 = pos - (double)c, w0 = 1.0 - w1;
     double ep[3], bp[3];
-    gather_eb<M>(eb, w0, w1, pc, ps, ep, bp, UniformFence());
+    gather_eb<M>(eb, w0, w1, pc, ps, ep, bp, fence);
     double gam_corr = 0.0;
     LaserAt la;
     if constexpr (PGC) {
@@ -999,8 +1018,8 @@ struct JDepMulti {
 
 // waves per SIMD the compiler is asked to fit: the vector form of modes 0..2
 // lands a few VGPRs above the 128 that allow four
-template <int M, bool PGC, bool MF>
-constexpr int dep_min_waves() { return !MF && !PGC ? (M <= 2 ? 4 : 3) : 1; }
+template <int M, bool PGC, bool MF, bool SINGLE>
+constexpr int dep_min_waves() { return !MF && !PGC ? (M <= 2 && !SINGLE ? 4 : 3) : 1; }
 
 // The current deposit's launch is bound by its longest wave and by the FP64
 // issue rate (420 FP64 instructions per 64 particles at modes 0..2), not by
@@ -1016,14 +1035,18 @@ constexpr int dep_min_waves() { return !MF && !PGC ? (M <= 2 ? 4 : 3) : 1; }
 // that profiles show the first-iteration launches, which always work, apart)
 // MF: the matrix form of the accumulation (mf_accumulate) instead of the
 // vector form (tile_accumulate); the same values up to the order of the sums
-template <int M, bool SPEC, int CPW, bool STD, bool PGC = false, bool MF = false>
-__global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF>())) void k_amjdeposit(const JDepMulti m)
+// SINGLE: species2d%amjdp, whose fields are staged in LDS from e and b
+// (SplitFields) in the packed layout
+template <int M, bool SPEC, int CPW, bool STD, bool PGC = false, bool MF = false, bool SINGLE = false>
+__global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF, SINGLE>())) void k_amjdeposit(const JDepMulti m)
 {
     const JDepArgs a = m.s[__builtin_amdgcn_readfirstlane(blockIdx.y)];
     constexpr int NM = 2 * M + 1;
     constexpr int NV = 8 * NM;
     constexpr int NF = dep_staged<NM, PGC>();   // staged field values per cell
     constexpr int CH = crowd_chunks<CPW>(), PT = crowd_parts<CPW>();
+    constexpr int NE = SINGLE ? 12 * NM : 1;
+    __shared__ double fe[CPW][NE];   // E and B at the two nodes (SINGLE)
     // the laser fields at the two nodes of each wave's cell (PGC)
     __shared__ double sf[CPW][NF];
     // the particle rows of the wave's products, per wave
@@ -1061,9 +1084,14 @@ __global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF>())) void k_amj
         rg.cell = d.x;
     }
     uniform_ptr eb;
-    double fv[(NF + 63) / 64];
+    double fv[(NF + 63) / 64], ev[(NE + 63) / 64];
     auto load_fields = [&](int c) {
         eb = (uniform_ptr)(a.eb + (size_t)(c + 1) * (6 * NM));
+        if constexpr (SINGLE) {
+#pragma unroll
+            for (int u = 0; u < (NE + 63) / 64; u++)
+                ev[u] = SplitFields<NM>{a.e, a.b, nm, ld, c + 1}[min(lane + 64 * u, NE - 1)];
+        }
         if constexpr (PGC) {
 #pragma unroll
             for (int u = 0; u < (NF + 63) / 64; u++)
@@ -1099,14 +1127,19 @@ __global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF>())) void k_amj
     dep_acc4 macc;
     double *const wrows = mrows + wave * ROWS;
     auto stage_fields = [&]() {
+        if constexpr (SINGLE) {
+#pragma unroll
+            for (int u = 0; u < (NE + 63) / 64; u++)
+                if (lane + 64 * u < NE) fe[wave][lane + 64 * u] = ev[u];
+        }
         if constexpr (PGC) {
 #pragma unroll
             for (int u = 0; u < (NF + 63) / 64; u++) {
                 const int l = lane + 64 * u;
                 if (l < NF) sf[wave][l] = fv[u];
             }
-            wave_lds_sync();
         }
+        if constexpr (SINGLE || PGC) wave_lds_sync();
     };
     // the wave's sums, value comp * NM + k of node ix to D0 and of node ix + 1 to D1
     auto store = [&](double *D0, double *D1) {
@@ -1148,14 +1181,21 @@ __global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF>())) void k_amj
         double x1 = X1[pc], x2 = X2[pc], pp1 = PP1[pc], pp2 = PP2[pc], pp3 = PP3[pc], qp = Q[pc];
         double psip = STD ? a.psi[pc] : 0.0;
         for (int k = 0; k < npass; k++, p += 64) {
-            // the fields are read anew for every pass (scalar cache) rather
-            // than held in registers
-            UniformFence()(eb);
+            // the fields are read anew for every pass (scalar cache or LDS)
+            // rather than held in registers
+            if constexpr (SINGLE) __asm__ volatile("" ::: "memory");
+            else UniformFence()(eb);
             const int pn = min(p + 64, pl);
             const double nx1 = X1[pn], nx2 = X2[pn], np1 = PP1[pn], np2 = PP2[pn], np3 = PP3[pn], nq = Q[pn];
             const double npsi = STD ? a.psi[pn] : 0.0;
             PartTerms<M> pt;
-            particle_terms<M, STD, PGC>(a, eb, sf[wave], c, p, p < p1, x1, x2, pp1, pp2, pp3, qp, psip, pt);
+            if constexpr (SINGLE) {
+                particle_terms<M, STD, PGC>(a, (const double *)fe[wave], NoFence(), sf[wave], c, p, p < p1, x1, x2, pp1,
+                                            pp2, pp3, qp, psip, pt);
+            } else {
+                particle_terms<M, STD, PGC>(a, eb, UniformFence(), sf[wave], c, p, p < p1, x1, x2, pp1, pp2, pp3, qp,
+                                            psip, pt);
+            }
             if constexpr (MF) {
                 mf_accumulate<M>(wrows, pt, lane, macc);
             } else {
@@ -1215,6 +1255,8 @@ static JDepArgs jdep_args(qpad_ctx *c, int s, int l, bool store_diag, bool repor
     a.store_diag = store_diag;
     a.cs = sp.cell_start;
     a.eb = c->eb;
+    a.e = c->f[QPAD_F_E];
+    a.b = c->f[QPAD_F_B];
     a.ar = c->f[QPAD_F_AR];
     a.ai = c->f[QPAD_F_AI];
     a.arg = c->f[QPAD_F_AR_GRAD];
@@ -1237,14 +1279,16 @@ static JDepArgs jdep_args(qpad_ctx *c, int s, int l, bool store_diag, bool repor
 }
 
 // the species of species-list entries in one launch (grid rows by list
-// entry), all of the push type STD, PGC names
+// entry), all of the push type STD, PGC names; l: the iteration, 0 a single
+// call (one workgroup shape: no result depends on it)
 template <bool STD, bool PGC>
 static int launch_jdep_list(qpad_ctx *c, const int *list, int n, int l, bool store_diag, bool timed, bool report)
 {
     const bool speculative = l >= 2;
     JDepMulti m;
     memset(&m, 0, sizeof(m));
-    const int cpw = c->dep_cells;
+    const bool single = l == 0;
+    const int cpw = single ? kDepWaves : c->dep_cells;
     int gx = 1;
     for (int i = 0; i < n; i++) {
         const int s = list[i];
@@ -1269,7 +1313,10 @@ static int launch_jdep_list(qpad_ctx *c, const int *list, int n, int l, bool sto
     } while (0)
 #define QPAD_DEP(MM)                                 \
     do {                                             \
-        if (cpw == 2) QPAD_DEP2(MM, 2);              \
+        if (single) {                                                                                              \
+            if (mf) hipLaunchKernelGGL((k_amjdeposit<MM, false, kDepWaves, STD, PGC, true, true>), grid, blk, 0, c->stream, m); \
+            else hipLaunchKernelGGL((k_amjdeposit<MM, false, kDepWaves, STD, PGC, false, true>), grid, blk, 0, c->stream, m);   \
+        } else if (cpw == 2) QPAD_DEP2(MM, 2);       \
         else if (cpw == 8) QPAD_DEP2(MM, 8);         \
         else QPAD_DEP2(MM, 4);                       \
     } while (0)
@@ -1354,6 +1401,7 @@ struct PushArgs {
     double idr, edge, qtmh, dt, qbm;
     double clamp;        // expansion-factor clamp of a sub-cycled push (0: none)
     const double *eb;    // the packed E and B of the slice
+    const double *e, *b; // the slice fields (single calls)
     const double *ar, *ai, *arg, *aig;   // laser envelope and gradients (PGC)
     double *x1, *x2, *p1, *p2, *p3, *gamma;   // pushed in place
     const double *psi;   // interpolated psi (standard pusher)
@@ -1376,7 +1424,8 @@ struct PushMulti {
 // same steps): the standard normalisation, the ponderomotive term in E with
 // the stored gamma, and the new gamma with gam_corr extrapolated half a step
 // in xi (the envelope's xi gradient).  Returns the new cell.
-template <int M, bool STD, bool PGC>
+// SINGLE: the fields from e and b (species2d%push, SplitFields).
+template <int M, bool STD, bool PGC, bool SINGLE>
 __device__ __forceinline__ uint32_t push_particle(const PushArgs &a, int64_t p)
 {
     const int nm = a.nm, ld = a.ld;
@@ -1389,7 +1438,10 @@ __device__ __forceinline__ uint32_t push_particle(const PushArgs &a, int64_t p)
     const int ix = ic + 1;
     const double w1 = pos - (double)ic, w0 = 1.0 - w1;
     double ep[3], bp[3];
-    gather_eb<M>(a.eb + (size_t)ix * (6 * (2 * M + 1)), w0, w1, pc, ps, ep, bp, NoFence());
+    if constexpr (SINGLE)
+        gather_eb<M>(SplitFields<2 * M + 1>{a.e, a.b, nm, ld, ix}, w0, w1, pc, ps, ep, bp, NoFence());
+    else
+        gather_eb<M>(a.eb + (size_t)ix * (6 * (2 * M + 1)), w0, w1, pc, ps, ep, bp, NoFence());
     double t = ep[0] * pc - ep[1] * ps;
     ep[1] = ep[0] * ps + ep[1] * pc;
     ep[0] = t;
@@ -1483,7 +1535,7 @@ __device__ __forceinline__ uint32_t push_particle(const PushArgs &a, int64_t p)
     return key;
 }
 
-template <int M, bool STD, bool PGC>
+template <int M, bool STD, bool PGC, bool SINGLE>
 __global__ __launch_bounds__(kSmallChunk) void k_push_count(const PushMulti m)
 {
     if ((int)blockIdx.y == m.n) {
@@ -1496,13 +1548,13 @@ __global__ __launch_bounds__(kSmallChunk) void k_push_count(const PushMulti m)
     const int64_t p = sort_element<kSmallChunk, 1>(0);
     uint32_t kv[1] = {(uint32_t)a.nr};
     if (p < a.s.n) {
-        if (p < a.s.cs[a.nr]) kv[0] = push_particle<M, STD, PGC>(a, p);
+        if (p < a.s.cs[a.nr]) kv[0] = push_particle<M, STD, PGC, SINGLE>(a, p);
         else a.s.key_w[p] = (uint32_t)a.nr;
     }
     chunk_hist<kSmallChunk, 1>(a.s, kv, lds);
 }
 
-template <int M, bool STD, bool PGC>
+template <int M, bool STD, bool PGC, bool SINGLE>
 __global__ __launch_bounds__(kPushThreads) void k_push(const PushMulti m)
 {
     if ((int)blockIdx.y == m.n) {
@@ -1517,7 +1569,7 @@ __global__ __launch_bounds__(kPushThreads) void k_push(const PushMulti m)
         a.s.key_w[p] = (uint32_t)a.nr;
         return;
     }
-    push_particle<M, STD, PGC>(a, p);
+    push_particle<M, STD, PGC, SINGLE>(a, p);
 }
 
 static PushArgs push_args(qpad_ctx *c, int s)
@@ -1534,6 +1586,8 @@ static PushArgs push_args(qpad_ctx *c, int s)
     a.clamp = c->clamp2d;
     a.qbm = sp.qbm;
     a.eb = c->eb;
+    a.e = c->f[QPAD_F_E];
+    a.b = c->f[QPAD_F_B];
     a.ar = c->f[QPAD_F_AR];
     a.ai = c->f[QPAD_F_AI];
     a.arg = c->f[QPAD_F_AR_GRAD];
@@ -1546,7 +1600,7 @@ static PushArgs push_args(qpad_ctx *c, int s)
 
 // the species of list entries (all of the push type STD, PGC names and all
 // in one sort form)
-template <bool STD, bool PGC>
+template <bool STD, bool PGC, bool SINGLE>
 static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &epi)
 {
     PushMulti m;
@@ -1580,8 +1634,9 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &
         time_begin(c, 1, &stop);
 #define QPAD_MOVE(MM)                                                                                       \
     do {                                                                                                    \
-        if (form == SORT_DIRECT) hipLaunchKernelGGL((k_push_count<MM, STD, PGC>), cg, blk, clds, c->stream, m); \
-        else hipLaunchKernelGGL((k_push<MM, STD, PGC>), pg, dim3(kPushThreads), 0, c->stream, m);            \
+        if (form == SORT_DIRECT)                                                                            \
+            hipLaunchKernelGGL((k_push_count<MM, STD, PGC, SINGLE>), cg, blk, clds, c->stream, m);           \
+        else hipLaunchKernelGGL((k_push<MM, STD, PGC, SINGLE>), pg, dim3(kPushThreads), 0, c->stream, m);    \
     } while (0)
         switch (c->g.M) {
         case 0: QPAD_MOVE(0); break;
@@ -1601,6 +1656,7 @@ static int launch_move_list(qpad_ctx *c, const int *list, int n, int form, int &
 
 // species s0 .. s1-1: one set of launches per push (the two PGC pushers push
 // alike) and sort form present, the first with slice epi's epilogue (0: none)
+template <bool SINGLE>
 static int launch_move_range(qpad_ctx *c, int s0, int s1, int epi)
 {
     for (int g = 0; g < 3; g++)
@@ -1610,16 +1666,16 @@ static int launch_move_range(qpad_ctx *c, int s0, int s1, int epi)
                 if (std::min(push_group(c->sp[s].cfg.push_type), 2) == g && sort_args(c, s).form == form)
                     list[n++] = s;
             if (!n) continue;
-            if (g == 0) QPAD_TRY((launch_move_list<false, false>(c, list, n, form, epi)));
-            else if (g == 1) QPAD_TRY((launch_move_list<true, false>(c, list, n, form, epi)));
-            else QPAD_TRY((launch_move_list<false, true>(c, list, n, form, epi)));
+            if (g == 0) QPAD_TRY((launch_move_list<false, false, SINGLE>(c, list, n, form, epi)));
+            else if (g == 1) QPAD_TRY((launch_move_list<true, false, SINGLE>(c, list, n, form, epi)));
+            else QPAD_TRY((launch_move_list<false, true, SINGLE>(c, list, n, form, epi)));
         }
     return epi > 0 ? launch_epilogue(c, epi) : 0;   // no particles
 }
 
-int launch_move(qpad_ctx *c, int s) { return launch_move_range(c, s, s + 1, 0); }
+int launch_move(qpad_ctx *c, int s) { return launch_move_range<true>(c, s, s + 1, 0); }
 
-int launch_move_all(qpad_ctx *c, int epi) { return launch_move_range(c, 0, c->nspecies, epi); }
+int launch_move_all(qpad_ctx *c, int epi) { return launch_move_range<false>(c, 0, c->nspecies, epi); }
 
 // ---------------------------------------------------------------------------
 // interp_psi_part2d (part2d_class.f03:2264-2305): the field psi at every

@@ -866,38 +866,6 @@ __global__ __launch_bounds__(kNodeThreads) void k_eperp(EperpArgs a)
     eb[2] = make_double2(bv[1], bv[2]);
 }
 
-// thread per (node i = 0..nr+1, mode array k), k fastest so that the stores
-// of a wave are one run: e and b into the packed fields (the fine-grained
-// calls, whose e and b come from separate solves; a thread per node with rows by
-// mode array before: 6.0 -> 5.2 us a call at M = 2)
-template <int NM>
-__global__ __launch_bounds__(64) void k_pack_eb(const double *e, const double *b, double *eb, int nr, int ld)
-{
-    const int nm = NM, t = blockIdx.x * blockDim.x + threadIdx.x, i = t / NM, k = t % NM;
-    if (i > nr + 1) return;
-    const double e0 = FX(e, 0, k, i), e1 = FX(e, 1, k, i), e2 = FX(e, 2, k, i);
-    const double b0 = FX(b, 0, k, i), b1 = FX(b, 1, k, i), b2 = FX(b, 2, k, i);
-    double2 *o = reinterpret_cast<double2 *>(eb + (size_t)t * 6);
-    o[0] = make_double2(e0, e1);
-    o[1] = make_double2(e2, b0);
-    o[2] = make_double2(b1, b2);
-}
-
-int launch_pack_eb(qpad_ctx *c)
-{
-    const dim3 grid((unsigned)(((c->g.nr + 2) * c->g.nm + 63) / 64)), blk(64);
-    const double *e = c->f[QPAD_F_E], *b = c->f[QPAD_F_B];
-    switch (c->g.M) {
-    case 0: hipLaunchKernelGGL(k_pack_eb<1>, grid, blk, 0, c->stream, e, b, c->eb, c->g.nr, c->g.ld); break;
-    case 1: hipLaunchKernelGGL(k_pack_eb<3>, grid, blk, 0, c->stream, e, b, c->eb, c->g.nr, c->g.ld); break;
-    case 2: hipLaunchKernelGGL(k_pack_eb<5>, grid, blk, 0, c->stream, e, b, c->eb, c->g.nr, c->g.ld); break;
-    case 3: hipLaunchKernelGGL(k_pack_eb<7>, grid, blk, 0, c->stream, e, b, c->eb, c->g.nr, c->g.ld); break;
-    default: hipLaunchKernelGGL(k_pack_eb<9>, grid, blk, 0, c->stream, e, b, c->eb, c->g.nr, c->g.ld); break;
-    }
-    QPAD_HIP_CHECK(hipGetLastError());
-    return 0;
-}
-
 int src_rows_host(int M, int nm) { return src_rows(M, nm); }
 
 // sources of the slice start (q_spe, the psi / Bz / Ez right-hand sides)

@@ -38,8 +38,6 @@ int launch_compare_only(qpad_ctx *c);
 // (k_solve), then b_spe, b, E_perp and the convergence maxima (k_bfields);
 // each returns at once once the iteration has converged
 int launch_iteration_fields(qpad_ctx *c, int j, int l);
-// the packed fields (qpad_ctx::eb) from the e and b slice fields
-int launch_pack_eb(qpad_ctx *c);
 // slice epilogue: cbq, e_spe, history copies, beam fields of slice j, the
 // J_perp predictor for the next slice
 int launch_epilogue(qpad_ctx *c, int j);
@@ -94,8 +92,9 @@ int launch_combine_q_rows(qpad_ctx *c, int sp, const DepRows &rows, double *out,
 int launch_chi_deposit_rows(qpad_ctx *c, int sp, const DepRows &rows);
 // l: predictor-corrector iteration of the slice (1-based; l >= 2 is a
 // speculative launch that first evaluates the convergence of iteration l-1
-// and returns at once when it has converged; l = 0 for a plain deposit);
-// timed: bracket the launch with the timing events of pool 0
+// and returns at once when it has converged; l = 0 for a single call, which
+// reads e and b themselves); timed: bracket the launch with the timing events
+// of pool 0
 int launch_amjdeposit(qpad_ctx *c, int sp, int l, bool store_diag, bool timed, bool report = false);
 // the same for every species in one launch (the workgroup rows are the
 // species); report: from species 0
@@ -104,7 +103,8 @@ int launch_amjdeposit_all(qpad_ctx *c, int l, bool store_diag, bool timed, bool 
 // convergence maximum pair each; at most kConvMaxBlocks)
 constexpr int kBfThreads = 64;
 inline int conv_blocks(int nr) { return (nr + 2 + kBfThreads - 1) / kBfThreads; }
-// push_u + push_x and the re-sort by the new cells (from the packed fields)
+// push_u + push_x and the re-sort by the new cells: one species from e and b
+// (a single call), or every species from the packed fields
 int launch_move(qpad_ctx *c, int sp);
 int launch_move_all(qpad_ctx *c, int epi);       // (and the epilogue of slice epi > 0) every species, one set of launches per pusher
 int launch_interp_psi(qpad_ctx *c, int sp);      // psi at the particles (standard pusher only)

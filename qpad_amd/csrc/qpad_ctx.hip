@@ -1305,7 +1305,6 @@ int qpad_species_amjdp(qpad_ctx *c, int32_t s, double dxi)
 {
     if (!c || s < 0 || s >= c->nspecies) return fail(QPAD_E_INVALID, "bad species");
     if (!(dxi > 0.0 && dxi < INFINITY)) return fail(QPAD_E_INVALID, "dxi must be > 0");
-    TRY(launch_pack_eb(c));
     c->dt2d = dxi;
     const int rc = launch_amjdeposit(c, s, 0, true, false);
     c->dt2d = c->g.dxi;
@@ -1398,7 +1397,6 @@ static int species_push(qpad_ctx *c, int32_t s, double dxi, double clamp)
 {
     if (!c || s < 0 || s >= c->nspecies) return fail(QPAD_E_INVALID, "bad species");
     if (!(dxi > 0.0 && dxi < INFINITY)) return fail(QPAD_E_INVALID, "dxi must be > 0");
-    TRY(launch_pack_eb(c));
     c->dt2d = dxi;
     c->clamp2d = clamp;
     int rc = launch_move(c, s);

@@ -148,7 +148,7 @@ struct qpad_ctx {
     int ncomp[QPAD_NFIELD];
     // E and B of the slice packed for the gathers of the current deposit and
     // the push: [node 0..nr+1][k][e_r, e_phi, e_z, b_r, b_phi, b_z]; written
-    // with e and b by the slice's field kernels (launch_pack_eb elsewhere)
+    // with e and b by the slice's field kernels (the single calls read e and b)
     double *eb;
     // histories (slices 0..nxi+1)
     double *h_psi, *h_e, *h_b, *h_b_spe, *h_e_spe, *h_cu, *h_q_spe, *h_q_beam, *h_b_beam;
