@@ -519,22 +519,138 @@ struct BDepArgs {
     double *h;   // q_beam history [s][nm][ld]
 };
 
-// Workgroup = 64 nodes of one history slice s = 1..nxi+1; a wave takes every
-// fourth group of 4 nodes that have particles, 16 particles of each node at a
-// time.  A node's sum is a chain over its particles, hundreds of times the
-// mean in a beam's core: a lane each does the root and the divisions of its
-// particle and leaves weight and phases in LDS, then a lane per node and mode
-// array adds them in particle order, so that the chain is 16 multiply-adds a
-// round.  A node's particles of a cell are consecutive: coalesced loads,
-// requested a round ahead (MI355X, one launch, a thread per node doing all of
-// its chain before: 262,144 particles in 256 x 256 cells 866 -> 116 us; 2^20 in
-// 4096 x 256 801 -> 127, in 2048 x 256 with modes 0..4 1116 -> 174).
+// Workgroup = 64 nodes of one history slice s = 1..nxi+1.  A node's sum is a
+// chain over its particles, hundreds of times the mean in a beam's core, none
+// for most nodes: lanes evaluate a node's particles (root, divisions) several
+// at a time and leave weight and phases in LDS, then a lane per node and mode
+// array adds them in particle order.  Particles are requested a round ahead.
+// - Tiles that no particle reaches only store.
+// - Sparse tiles (at most kBDepSparse particles reach them): a wave takes 16
+//   nodes, 4 particles each a round, its four cells' one after the other.
+// - Others: a wave takes every fourth group of 4 nodes that have particles, 16
+//   particles of each node and cell a round, so that the chain is 16
+//   multiply-adds a round.
+// MI355X, one launch, a thread per node doing all of its chain -> every tile in
+// the last form -> now: 262,144 particles in 256 x 256 cells (all of it in
+// the last form) 1766 -> 191 -> 191 us; 2^20 in 4096 x 256 913 -> 131 -> 115, in 2048 x
+// 256 with modes 0..4 350 -> 175 -> 112; 2^14 in 4096 x 256 28 -> 48 -> 26, 2^12
+// in 1024 x 512 14.7 -> 28.4 -> 15.7, 2^16 all over 8192 x 128 31 -> 129 -> 39.
+// The line at 512: with 256 the third is 124 us, with 1024 99 but 2^20 in 2048
+// x 256 (core of a beam) 196 against 184.  From modes 0..2 up five waves per
+// SIMD are asked for (94 VGPRs instead of 107, no spill): tiles with little
+// work wait on latency.
 constexpr int kBDepNodes = 64, kBDepGroup = 4, kBDepAhead = 64 / kBDepGroup;
 constexpr int kBDepPitch = kBDepGroup * (kBDepAhead + 1);   // padded rows of the groups' stage
+constexpr int kBDepSparse = 512;
 static_assert(kMaxNm <= kBDepAhead, "a lane per node of the group and mode array");
 
+// a particle's weight on a node (side dk of its xi cell mm, dj of its r cell
+// nn) to w, and its charge times e^{-im phi} of mode array k to h[k * pitch].
+// The fused multiply-adds are written out, so that both forms give the same
+// bits.
 template <int M>
-__global__ __launch_bounds__(4 * 64) void k_beam_qdeposit(BDepArgs a)
+__device__ __forceinline__ void bdep_terms(const BDepArgs &a, double x1, double x2, double x3, double q, int mm, int nn,
+                                           int dk, int dj, double &w, double *h)
+{
+#pragma clang fp contract(off)
+    const double r = sqrt(fma(x2, x2, x1 * x1)), pr = r * a.idr;
+    const double ph0r = x1 / pr * a.idr, ph0i = -x2 / pr * a.idr;
+    const double wr = fma(r, a.idr, -(double)nn), wz = fma(x3, a.idz, -(double)mm);
+    const double wrj = dj ? wr : 1.0 - wr, wzk = dk ? wz : 1.0 - wz;
+    double phr = 1.0 * q, phi = 0.0;
+    w = wrj * wzk;
+    h[0] = phr;
+#pragma unroll
+    for (int m = 1; m <= M; m++) {
+        const double tr = fma(phr, ph0r, -(phi * ph0i)), ti = fma(phr, ph0i, phi * ph0r);
+        phr = tr;
+        phi = ti;
+        h[(2 * m - 1) * kBDepPitch] = phr;
+        h[2 * m * kBDepPitch] = phi;
+    }
+}
+
+__device__ __forceinline__ void bdep_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// where a sparse node's particles are: those of its cells d = 0..3 one after
+// the other, cell d's up to number t_d+1, at b_d + the number
+struct BDepNode {
+    int t1, t2, t3, t4, b0, b1, b2, b3;
+    // particle j, clamped into the node's; d its cell
+    __device__ __forceinline__ int at(int j, int &d) const
+    {
+        j = min(j, t4 - 1);
+        const int lo = j < t1 ? b0 : b1, hi = j < t3 ? b2 : b3;
+        d = (j >= t1) + (j >= t2) + (j >= t3);
+        return t4 > 0 ? j + (j < t2 ? lo : hi) : 0;
+    }
+};
+
+// the sparse form: sums of the nodes 16 wave .. 16 wave + 15 of the tile
+template <int M>
+__device__ __forceinline__ void bdep_sparse(const BDepArgs &a, const double *px1, const double *px2, const double *px3,
+                                            const double *pq, const int32_t *cs, int s, int i0, int wave,
+                                            int lane, double (*st)[kBDepPitch], double (*res)[kBDepNodes])
+{
+    constexpr int NM = 2 * M + 1, SLOTS = (NM + 3) / 4, W = 4;
+    const int gn = lane / W, gj = lane % W, node = 16 * wave + gn;
+    // lane gj of a node looks up its cell d = gj
+    const int mm = s - 1 - (gj >> 1), nn = i0 + node - 1 - (gj & 1);
+    const bool in = mm >= 0 && mm < a.nxi && nn >= 0 && nn < a.nr;
+    const int cell = in ? mm * a.nr + nn : 0;
+    const int f0 = cs[cell], f1 = cs[cell + 1];
+    const int first = in ? f0 : 0, count = in ? f1 - f0 : 0, at = W * gn;
+    BDepNode n;
+    n.b0 = __shfl(first, at, 64);
+    n.t1 = __shfl(count, at, 64);
+    n.b1 = __shfl(first, at + 1, 64) - n.t1;
+    n.t2 = n.t1 + __shfl(count, at + 1, 64);
+    n.b2 = __shfl(first, at + 2, 64) - n.t2;
+    n.t3 = n.t2 + __shfl(count, at + 2, 64);
+    n.b3 = __shfl(first, at + 3, 64) - n.t3;
+    n.t4 = n.t3 + __shfl(count, at + 3, 64);
+    int most = n.t4;
+    for (int d = W; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d, 64));
+    most = __builtin_amdgcn_readfirstlane(most);
+    double acc[SLOTS];
+#pragma unroll
+    for (int v = 0; v < SLOTS; v++) acc[v] = 0.0;
+    int d = 0;
+    int e = n.at(gj, d);
+    double x1 = px1[e], x2 = px2[e], x3 = px3[e], q = pq[e];
+    for (int o = 0; o < most; o += W) {
+        const double y1 = x1, y2 = x2, y3 = x3, yq = q;
+        const int dk = d >> 1, dj = d & 1;
+        e = n.at(o + W + gj, d);
+        x1 = px1[e];
+        x2 = px2[e];
+        x3 = px3[e];
+        q = pq[e];
+        bdep_terms<M>(a, y1, y2, y3, yq, s - 1 - dk, i0 + node - 1 - dj, dk, dj, st[NM][lane], &st[0][lane]);
+        bdep_wave_sync();
+#pragma unroll
+        for (int u = 0; u < W; u++) {
+            const double w = st[NM][W * gn + u];
+#pragma unroll
+            for (int v = 0; v < SLOTS; v++) {
+                const double next = fma(w, st[min(gj + W * v, NM - 1)][W * gn + u], acc[v]);
+                acc[v] = o + u < n.t4 ? next : acc[v];
+            }
+        }
+        bdep_wave_sync();
+    }
+#pragma unroll
+    for (int v = 0; v < SLOTS; v++)
+        if (gj + W * v < NM) res[gj + W * v][node] = acc[v];
+}
+
+template <int M>
+__global__ __launch_bounds__(4 * 64, (M >= 2 ? 5 : 1)) void k_beam_qdeposit(BDepArgs a)
 {
     constexpr int NM = 2 * M + 1, SLOTS = (NM + 3) / 4;
     __shared__ double res[NM][kBDepNodes];
@@ -549,76 +665,70 @@ __global__ __launch_bounds__(4 * 64) void k_beam_qdeposit(BDepArgs a)
 #pragma unroll
     for (int u = 0; u < SLOTS; u++) tot[u] = 0.0;
     for (int b = 0; b < a.nbeams; b++) {
-        const double *px1 = a.x1[b], *px2 = a.x2[b], *px3 = a.x3[b], *pq = a.q[b];
-        // particles of node i's four neighbouring cells: xi cell mm = s-1-dk,
-        // r cell nn = i-1-dj, d = 2 dk + dj
-        int r0[4], r1[4];
+        // the tile's cells are one run in each of the two xi cells
+        const int lo = max(i0 - 2, 0), hi = min(i0 + kBDepNodes - 2, nr - 1);
+        int reach = 0;   // particles of them
 #pragma unroll
-        for (int d = 0; d < 4; d++) {
-            const int mm = s - 1 - (d >> 1), nn = i - 1 - (d & 1);
-            const bool in = mm >= 0 && mm < nxi && nn >= 0 && nn < nr;
-            const int cell = in ? mm * nr + nn : 0;
-            const int c0 = a.cs[b][cell], c1 = a.cs[b][cell + 1];
-            r0[d] = in ? c0 : 0;
-            r1[d] = in ? c1 : 0;
+        for (int dk = 0; dk < 2; dk++) {
+            const int mm = s - 1 - dk;
+            if (mm >= 0 && mm < nxi && lo <= hi) reach += a.cs[b][mm * nr + hi + 1] - a.cs[b][mm * nr + lo];
         }
-        const uint64_t full = __ballot(r1[0] > r0[0] || r1[1] > r0[1] || r1[2] > r0[2] || r1[3] > r0[3]);
-        for (int g = wave; g < kBDepNodes / kBDepGroup; g += 4) {
-            const int node = kBDepGroup * g + gn;
-            double acc = 0.0;
-            if ((full >> (kBDepGroup * g)) & ((1u << kBDepGroup) - 1)) {
+        if (reach == 0) continue;
+        const double *px1 = a.x1[b], *px2 = a.x2[b], *px3 = a.x3[b], *pq = a.q[b];
+        if (reach <= kBDepSparse) {
+            bdep_sparse<M>(a, px1, px2, px3, pq, a.cs[b], s, i0, wave, lane, st, res);
+        } else {
+            // particles of node i's four neighbouring cells: xi cell mm = s-1-dk,
+            // r cell nn = i-1-dj, d = 2 dk + dj
+            int r0[4], r1[4];
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                const int mm = s - 1 - (d >> 1), nn = i - 1 - (d & 1);
+                const bool in = mm >= 0 && mm < nxi && nn >= 0 && nn < nr;
+                const int cell = in ? mm * nr + nn : 0;
+                const int c0 = a.cs[b][cell], c1 = a.cs[b][cell + 1];
+                r0[d] = in ? c0 : 0;
+                r1[d] = in ? c1 : 0;
+            }
+            const uint64_t full = __ballot(r1[0] > r0[0] || r1[1] > r0[1] || r1[2] > r0[2] || r1[3] > r0[3]);
+            for (int g = wave; g < kBDepNodes / kBDepGroup; g += 4) {
+                const int node = kBDepGroup * g + gn;
+                double acc = 0.0;
+                if ((full >> (kBDepGroup * g)) & ((1u << kBDepGroup) - 1)) {
 #pragma unroll 1
-                for (int d = 0; d < 4; d++) {
-                    const int dk = d >> 1, dj = d & 1, mm = s - 1 - dk, nn = i0 + node - 1 - dj;
-                    const int c0 = __shfl(d == 0 ? r0[0] : d == 1 ? r0[1] : d == 2 ? r0[2] : r0[3], node, 64);
-                    const int c1 = __shfl(d == 0 ? r1[0] : d == 1 ? r1[1] : d == 2 ? r1[2] : r1[3], node, 64);
-                    int most = c1 - c0;
-                    most = max(most, __shfl_xor(most, 16, 64));
-                    most = __builtin_amdgcn_readfirstlane(max(most, __shfl_xor(most, 32, 64)));
-                    if (most == 0) continue;
-                    int e = max(min(c0 + gj, c1 - 1), 0);
-                    double x1 = px1[e], x2 = px2[e], x3 = px3[e], q = pq[e];
-                    for (int o = 0; o < most; o += kBDepAhead) {
-                        const double y1 = x1, y2 = x2, y3 = x3, yq = q;
-                        e = max(min(c0 + o + kBDepAhead + gj, c1 - 1), 0);
-                        x1 = px1[e];
-                        x2 = px2[e];
-                        x3 = px3[e];
-                        q = pq[e];
-                        const double pr = __dmul_rn(bradius(y1, y2), a.idr);
-                        const double pz = y3 * a.idz;
-                        const double ph0r = y1 / pr * a.idr, ph0i = -y2 / pr * a.idr;
-                        const double wr = pr - (double)nn, wz = pz - (double)mm;
-                        const double wrj = dj ? wr : 1.0 - wr, wzk = dk ? wz : 1.0 - wz;
-                        double phr = 1.0 * yq, phi = 0.0;
-                        const int at = gn * (kBDepAhead + 1);
-                        st[NM][at + gj] = wrj * wzk;
-                        st[0][at + gj] = phr;
+                    for (int d = 0; d < 4; d++) {
+                        const int dk = d >> 1, dj = d & 1, mm = s - 1 - dk, nn = i0 + node - 1 - dj;
+                        const int c0 = __shfl(d == 0 ? r0[0] : d == 1 ? r0[1] : d == 2 ? r0[2] : r0[3], node, 64);
+                        const int c1 = __shfl(d == 0 ? r1[0] : d == 1 ? r1[1] : d == 2 ? r1[2] : r1[3], node, 64);
+                        int most = c1 - c0;
+                        most = max(most, __shfl_xor(most, 16, 64));
+                        most = __builtin_amdgcn_readfirstlane(max(most, __shfl_xor(most, 32, 64)));
+                        if (most == 0) continue;
+                        int e = max(min(c0 + gj, c1 - 1), 0);
+                        double x1 = px1[e], x2 = px2[e], x3 = px3[e], q = pq[e];
+                        for (int o = 0; o < most; o += kBDepAhead) {
+                            const double y1 = x1, y2 = x2, y3 = x3, yq = q;
+                            e = max(min(c0 + o + kBDepAhead + gj, c1 - 1), 0);
+                            x1 = px1[e];
+                            x2 = px2[e];
+                            x3 = px3[e];
+                            q = pq[e];
+                            const int at = gn * (kBDepAhead + 1);
+                            bdep_terms<M>(a, y1, y2, y3, yq, mm, nn, dk, dj, st[NM][at + gj], &st[0][at + gj]);
+                            bdep_wave_sync();
+                            const double *w_ = &st[NM][at], *h_ = &st[min(gj, NM - 1)][at];
+                            const int n = c1 - c0 - o;
 #pragma unroll
-                        for (int m = 1; m <= M; m++) {
-                            const double tr = phr * ph0r - phi * ph0i, ti = phr * ph0i + phi * ph0r;
-                            phr = tr;
-                            phi = ti;
-                            st[2 * m - 1][at + gj] = phr;
-                            st[2 * m][at + gj] = phi;
+                            for (int u = 0; u < kBDepAhead; u++) {
+                                const double next = fma(w_[u], h_[u], acc);
+                                acc = u < n ? next : acc;
+                            }
+                            bdep_wave_sync();
                         }
-                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                        __builtin_amdgcn_wave_barrier();
-                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                        const double *w_ = &st[NM][at], *h_ = &st[min(gj, NM - 1)][at];
-                        const int n = c1 - c0 - o;
-#pragma unroll
-                        for (int u = 0; u < kBDepAhead; u++) {
-                            const double next = acc + w_[u] * h_[u];
-                            acc = u < n ? next : acc;
-                        }
-                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                        __builtin_amdgcn_wave_barrier();
-                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                     }
                 }
+                if (gj < NM) res[gj][node] = acc;
             }
-            if (gj < NM) res[gj][node] = acc;
         }
         __syncthreads();
         // axis and 1/r for slices 1..nzp (part3d_class.f03:315-351); wave w
