@@ -449,8 +449,8 @@ int qpad_set_beam(qpad_ctx *ctx, int32_t ib, int64_t n, const double *x1,
    sampled on the first predictor-corrector iteration of every slice (which
    always does work; events around every launch would slow the step):
    which = 0: plasma current deposit (amjdeposit), 1: the plasma push launches
-   (every slice, every species with particles; the launch also counts the
-   cells for the re-sort where the particles are few, and the slice's first
+   (every slice, one per pusher of the species with particles; they also count
+   the cells for the re-sort where the particles are few, and the slice's first
    one holds the slice's epilogue unless the learned seed is on), 2: the field
    sources and solves of the first iteration.  Returns the summed milliseconds
    and the number of timed launches since the last reset. */

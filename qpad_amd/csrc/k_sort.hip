@@ -128,14 +128,10 @@ int sort_workspace(int64_t npmax, int nr, size_t *hist_ints)
     return 0;
 }
 
-SortArgs sort_args(qpad_ctx *c, int s)
+int sort_form(qpad_ctx *c, int s)
 {
-    Species &sp = c->sp[s];
-    const int64_t n = sp.npp;
-    SortArgs a;
-    memset(&a, 0, sizeof(a));
-    a.n = n;
-    a.nb = c->g.nr + 1;
+    const int64_t n = c->sp[s].npp;
+    const int nr = c->g.nr, nb = nr + 1;
     // direct: push and re-sort, us a slice, chunks of 2048 with the scan launch
     // -> direct: 4096 particles in 256 cells 24.1 -> 11.7, 21189 in 1009 23.4 ->
     // 15.5, 24576 in 768 27 -> 19.5 (the sum over the chunks grows with chunks x
@@ -146,9 +142,19 @@ SortArgs sort_args(qpad_ctx *c, int s)
     // histogram costs more than the shorter chunks give: 393216 in 512 23.6 ->
     // 23.6, in 2048 24.2 -> 25.2, in 4096 25.7 -> 28.3; 196608 in 8192 26.0 -> 28.4
     const int64_t small = (n + kSmallChunk - 1) / kSmallChunk, mid = (n + kMidChunk - 1) / kMidChunk;
-    if (a.nb <= kDirectBins && small <= kDirectChunks && small * a.nb <= kDirectWork) a.form = SORT_DIRECT;
-    else if (n <= kMidMax && mid * c->g.nr <= kMidWork) a.form = SORT_MID;
-    else a.form = SORT_LARGE;
+    if (nb <= kDirectBins && small <= kDirectChunks && small * nb <= kDirectWork) return SORT_DIRECT;
+    return n <= kMidMax && mid * nr <= kMidWork ? SORT_MID : SORT_LARGE;
+}
+
+SortArgs sort_args(qpad_ctx *c, int s, int form)
+{
+    Species &sp = c->sp[s];
+    const int64_t n = sp.npp;
+    SortArgs a;
+    memset(&a, 0, sizeof(a));
+    a.n = n;
+    a.nb = c->g.nr + 1;
+    a.form = form;
     const int chunk = a.form == SORT_LARGE ? kSortChunk : a.form == SORT_MID ? kMidChunk : kSmallChunk;
     a.nchunks = (int)((n + chunk - 1) / chunk);
     a.key = sp.key;
@@ -220,7 +226,7 @@ int launch_sort(qpad_ctx *c, int s)
 {
     SortMulti m;
     memset(&m, 0, sizeof(m));
-    m.s[0] = sort_args(c, s);
+    m.s[0] = sort_args(c, s, sort_form(c, s));
     QPAD_TRY(launch_sort_list(c, m, 1, false));
     sort_swap(c->sp[s]);
     return 0;

@@ -106,7 +106,7 @@ inline int conv_blocks(int nr) { return (nr + 2 + kBfThreads - 1) / kBfThreads; 
 // push_u + push_x and the re-sort by the new cells: one species from e and b
 // (a single call), or every species from the packed fields
 int launch_move(qpad_ctx *c, int sp);
-int launch_move_all(qpad_ctx *c, int epi);       // (and the epilogue of slice epi > 0) every species, one set of launches per pusher
+int launch_move_all(qpad_ctx *c, int epi);       // and the epilogue of slice epi > 0: a push launch per pusher, one sort
 int launch_interp_psi(qpad_ctx *c, int sp);      // psi at the particles (standard pusher only)
 int launch_add_qn_into_qspe(qpad_ctx *c, int sp);
 // per-species charge (species2d%q, cbq): q of species sp from its charge

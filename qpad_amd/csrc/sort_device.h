@@ -33,7 +33,7 @@
 
 namespace qpad {
 
-// the forms, by the number of particles (sort_args):
+// the forms, by the number of particles (sort_form):
 //   direct  chunks of kSmallChunk, no scan launch, counted by the push;
 //   mid     chunks of kMidChunk;
 //   large   chunks of kSortChunk (fewer histogram rows).
@@ -435,7 +435,10 @@ __device__ __forceinline__ bool scatter_positions(const SortArgs &a, const uint3
 }
 
 // ---- host side (k_sort.hip) ----
-SortArgs sort_args(qpad_ctx *c, int s);
+// the form of species s by itself (SORT_LARGE takes every count)
+int sort_form(qpad_ctx *c, int s);
+// its arguments in that form or a more demanding species' (SORT_* below it)
+SortArgs sort_args(qpad_ctx *c, int s, int form);
 struct SortMulti {
     SortArgs s[kMaxSpecies];
 };

@@ -11,6 +11,7 @@ removed.  The order is exact: by cell, then by the order given."""
 import numpy as np
 import pytest
 
+import twin
 from qpad_amd import Simulation, configs
 
 pytestmark = pytest.mark.gpu
@@ -49,22 +50,47 @@ def test_sort_is_stable_and_complete(nr, n, spread):
     sim.close()
 
 
-@pytest.mark.parametrize("ppc,direct", [((2, 16), True), ((4, 130), True), ((4, 260), False)])
-def test_push_forms_keep_the_sorted_order(ppc, direct):
-    """both push forms leave the particles grouped by cell, each cell in the
-    order its particles had before (no particle lost or doubled)"""
-    sim = Simulation(configs.small(nr=64, nxi=40, max_mode=1, ppc=ppc, total_num=1 << 12, offset_x=0.02))
-    assert (64 * ppc[0] * ppc[1] <= 120 * 512) == direct
+@pytest.mark.parametrize("ppc,ion_ppc", [((2, 16), None), ((4, 130), None), ((4, 260), None), ((4, 260), (1, 3)),
+                                         ((1, 3), (4, 260))])
+def test_push_forms_keep_the_sorted_order(ppc, ion_ppc):
+    """every push and sort leaves the particles grouped by their new cell, each
+    cell in the order its particles had before, and drops exactly those that
+    the oracle's push takes out of the box (64 cells: up to 4 x 130 per cell in
+    the direct form, 4 x 260 past it, alone and beside a species of few)"""
+    sim = Simulation(configs.small(nr=64, nxi=40, max_mode=1, ppc=ppc, total_num=1 << 12, offset_x=0.02,
+                                   ions=ion_ppc is not None, ion_ppc=ion_ppc))
+    g = sim.grid
+    o = twin.make_twin(sim)
     sim.step3d_begin()
-    n0 = sim.spe[0].count()
-    for j in range(1, 31):
+    o.step_begin()
+    rng = np.random.default_rng(3)
+    # momenta that take some particles out of the box in every slice
+    for sp in sim.spe:
+        p = sp.get()
+        for k in ("p1", "p2", "p3"):
+            p[k] = 0.4 * rng.standard_normal(len(p[k]))
+        p["gamma"] = np.sqrt(1.0 + p["p1"] ** 2 + p["p2"] ** 2 + p["p3"] ** 2)
+        sp.set(p)
+    lost = 0
+    for j in range(1, 5):
+        before = [sp.get()["id"] for sp in sim.spe]
+        twin.sync_slice_inputs(sim, o, j)
         sim.slice(j)
-    p = sim.spe[0].get()
-    c = np.floor(np.hypot(p["x1"], p["x2"]) / sim.grid.dr).astype(int)
-    assert np.all(np.diff(c) >= 0) and c.max() < 64
-    assert len(np.unique(p["id"])) == len(p["id"]) <= n0
-    assert np.all(np.isfinite(p["gamma"])) and np.max(np.abs(p["p1"])) > 1e-3
+        o.slice(j)
+        for s, sp in enumerate(sim.spe):
+            p = sp.get()
+            kept = np.array(o.species(s)["id"])
+            assert np.array_equal(np.sort(p["id"]), np.sort(kept)), (j, s)
+            assert len(np.unique(p["id"])) == len(p["id"])
+            lost += len(before[s]) - len(kept)
+            c = (np.hypot(p["x1"], p["x2"]) / g.dr).astype(int)
+            assert np.all(np.diff(c) >= 0) and c.max() < g.nr
+            place = np.empty(before[s].max() + 1, dtype=int)
+            place[before[s]] = np.arange(len(before[s]))
+            assert np.array_equal(p["id"], p["id"][np.lexsort((place[p["id"]], c))]), (j, s)
+    assert lost > 0
     sim.close()
+    o.close()
 
 
 def test_species_without_particles_on_a_large_grid():
