@@ -248,8 +248,10 @@ struct QDepArgs {
 // same for every shape.
 constexpr int kDepSub = 4;
 constexpr int kDepPart = kDepChunk / kDepSub;
-// at most this many workgroups walk the crowded list
-constexpr int kCrowdGroups = 256;
+// at most this many workgroups walk the crowded list (on few cells all of
+// them may be on it, and fewer would walk it in rounds: 512 per cell in 1024
+// cells, M = 0, 7.2 ms with 512, 5.5 with 1024)
+inline int crowd_groups(int nr) { return nr <= kDepFewCells ? kDepFewCells : 256; }
 
 template <int CPW>
 constexpr int crowd_chunks() { return CPW >= 2 * kDepSub ? CPW / kDepSub : 1; }   // chunks of a workgroup at once
@@ -299,7 +301,7 @@ inline int dep_grid(int nr, int64_t npp, int first, int cpw)
 {
     const int chunks = (int)std::min<int64_t>(npp / (first + 1) + npp / kDepChunk, 1 << 20);
     const int per = cpw >= 2 * kDepSub ? cpw / kDepSub : 1;
-    return (nr + cpw - 1) / cpw + std::min((chunks + per - 1) / per, kCrowdGroups);
+    return (nr + cpw - 1) / cpw + std::min((chunks + per - 1) / per, crowd_groups(nr));
 }
 
 // the arguments of every species of one launch (workgroup rows by species)

@@ -603,9 +603,15 @@ static int species_create(qpad_ctx *c, const qpad_species_cfg *cfg, const qpad_n
     if (!rc) rc = dalloc(&sp.P1, (size_t)c->g.nr * 8 * c->g.nm);
     sp.n_ov_max = (int)(sp.npmax / kDepChunk + 1);
     // a wave takes cells of up to twice the injected particles per cell (at
-    // least four passes, at most one chunk)
+    // least four passes, at most one chunk); on a few cells only up to four
+    // passes, since their waves leave the chip idle (MI355X, all deposits of
+    // 128 slices, ms, a wave for a whole cell's injected particles -> four:
+    // 1024 per cell in 512 cells, M = 1, 9.06 -> 6.52, 512 in 1024, M = 0,
+    // 6.10 -> 5.53, 256 in 512, M = 4, 7.06 -> 6.30; in 2048 cells, M = 2,
+    // 7.08 -> 8.45)
     const int64_t per_cell = (int64_t)cfg->ppc1 * cfg->ppc2 * cfg->num_theta;
-    sp.dep_first = (int)std::min<int64_t>(std::max<int64_t>((2 * per_cell + 63) / 64 * 64, kDepFirstMin), kDepChunk);
+    sp.dep_first = c->g.nr <= kDepFewCells ? kDepFirstMin :
+        (int)std::min<int64_t>(std::max<int64_t>((2 * per_cell + 63) / 64 * 64, kDepFirstMin), kDepChunk);
     sp.n_crowd_max = (int)(sp.npmax / (sp.dep_first + 1) + sp.npmax / kDepChunk + 1);
     if (!rc) rc = dalloc(&sp.ov_start, (size_t)c->g.nr + 2);
     if (!rc) rc = dalloc(&sp.ov_desc, (size_t)sp.n_crowd_max);

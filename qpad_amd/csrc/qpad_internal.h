@@ -29,6 +29,9 @@ constexpr int kDepWaves = 4;         // default radial cells (waves) per deposit
 // holds more than Species::dep_first particles
 constexpr int kDepChunk = 1024;
 constexpr int kDepFirstMin = 256;
+// up to this many cells a wave per cell is at most one per SIMD, and cells of
+// more than kDepFirstMin particles are always shared
+constexpr int kDepFewCells = 1024;
 
 // field kinds (source/param.f03:75-84)
 enum { FK_PSI = 0, FK_EZ = 1, FK_BZ = 2, FK_BT = 3, FK_BPLUS = 4, FK_BMINUS = 5, FK_N = 6 };
