@@ -1018,10 +1018,13 @@ struct JDepMulti {
     JDepArgs s[kMaxSpecies];
 };
 
-// waves per SIMD the compiler is asked to fit: the vector form of modes 0..2
-// lands a few VGPRs above the 128 that allow four
+// waves per SIMD the compiler is asked to fit, without a spill: modes 0..1 of
+// the vector form take 92..128 VGPRs, modes 0..2 136.  Forced under 128, modes
+// 0..2 spill 6..12 VGPRs, and four waves give what the spills take: 524,288
+// particles in 4096 cells, first / later iterations, 20.4 / 14.8 us, with
+// three 19.9 / 15.0; 2^20 in 8192 29.7 / 23.2 and 29.0 / 23.2.
 template <int M, bool PGC, bool MF, bool SINGLE>
-constexpr int dep_min_waves() { return !MF && !PGC ? (M <= 2 && !SINGLE ? 4 : 3) : 1; }
+constexpr int dep_min_waves() { return !MF && !PGC ? (M <= 1 ? 4 : M >= 3 && SINGLE ? 2 : 3) : 1; }
 
 // The current deposit's launch is bound by its longest wave and by the FP64
 // issue rate (420 FP64 instructions per 64 particles at modes 0..2), not by
@@ -1056,6 +1059,7 @@ __global__ __launch_bounds__(64 * CPW, (dep_min_waves<M, PGC, MF, SINGLE>())) vo
     __shared__ __align__(16) double mrows[CPW * ROWS];
     // the part sums of crowded chunks
     __shared__ double comb[CH][kDepSub][2 * NV];
+    static_assert(sizeof(double) * (CPW * (NE + NF + ROWS) + CH * kDepSub * 2 * NV) <= 160 * 1024, "LDS of a CU");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nm = a.nm, ld = a.ld;
