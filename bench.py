@@ -22,9 +22,11 @@ reported beside it.  `batch_c4` times the C4 scan (16 independent
 instances) stepped one after another and as one batch (eager and graph).
 """
 import argparse
+import hashlib
 import json
 import multiprocessing as mp
 import os
+import re
 import sys
 import tempfile
 import time
@@ -91,20 +93,32 @@ def deck_for(name):
     return {"c1": configs.c1, "c2": configs.c2, "c3": configs.c3}[name]()
 
 
-def measured_traffic(workload, max_mode):
+def kernel_source_hash(root=ROOT):
+    """Hash of the deposit kernels' sources without comments and blanks: what
+    a traffic summary was measured on."""
+    h = hashlib.sha256()
+    for name in ("k_plasma.hip", "wave_reduce.h", "conv.h", "qpad_internal.h"):
+        with open(os.path.join(root, "qpad_amd", "csrc", name)) as f:
+            h.update(re.sub(r"\s+", "", re.sub(r"//[^\n]*", "", f.read())).encode())
+    return h.hexdigest()[:16]
+
+
+def measured_traffic(workload, max_mode, root=ROOT):
     """HBM bytes per launch of the first-iteration deposit from the committed
     rocprofv3 FETCH_SIZE / WRITE_SIZE summary (calibrated against a copy of
-    known size), or None when no summary covers this workload."""
-    path = os.path.join(ROOT, "profiles", f"k_amjdeposit_{workload}_hbm_traffic.txt")
+    known size), or None when no summary covers this workload or the summary
+    was measured on another kernel than the present one."""
+    path = os.path.join(root, "profiles", f"k_amjdeposit_{workload}_hbm_traffic.txt")
     if not os.path.exists(path):
         return None
-    text = open(path).read()
+    with open(path) as f:
+        text = f.read()
     if f"k_amjdeposit<{max_mode}, false" not in text:
         return None
-    for line in text.splitlines():
-        if line.startswith("traffic_bytes_per_launch:"):
-            return float(line.split(":", 1)[1])
-    return None
+    key = dict(re.findall(r"^(kernel_source|traffic_bytes_per_launch): (\S+)$", text, re.M))
+    if key.get("kernel_source") != kernel_source_hash(root) or "traffic_bytes_per_launch" not in key:
+        return None
+    return float(key["traffic_bytes_per_launch"])
 
 
 def algorithmic_bytes_per_step(grid, np_per_slice, iters, nbeam):

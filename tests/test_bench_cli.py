@@ -31,3 +31,29 @@ def test_options_parse():
     finally:
         sys.argv = argv
     assert a.only_c4 and a.c4_eager == "eager_single" and a.steps == 2 and a.no_cpu and a.gpus == 1
+
+
+def test_traffic_of_another_kernel_is_not_reported(tmp_path):
+    """the committed counter summary is printed only for the kernel it was
+    measured on: no figure once the deposit's source is another, or the
+    summary does not say which it was; comments do not matter"""
+    sys.path.insert(0, ROOT)
+    import bench
+    src = tmp_path / "qpad_amd" / "csrc"
+    src.mkdir(parents=True)
+    for name in ("k_plasma.hip", "wave_reduce.h", "conv.h", "qpad_internal.h"):
+        (src / name).write_text("int kernel;  // " + name + "\n")
+    (tmp_path / "profiles").mkdir()
+    summary = tmp_path / "profiles" / "k_amjdeposit_c2_hbm_traffic.txt"
+    head = "of k_amjdeposit<2, false, 4>\n"
+    assert bench.measured_traffic("c2", 2, str(tmp_path)) is None
+    summary.write_text(head + "traffic_bytes_per_launch: 41387494\n")
+    assert bench.measured_traffic("c2", 2, str(tmp_path)) is None
+    summary.write_text(head + f"kernel_source: {bench.kernel_source_hash(str(tmp_path))}\n"
+                       "traffic_bytes_per_launch: 41387494\n")
+    assert bench.measured_traffic("c2", 2, str(tmp_path)) == 41387494.0
+    assert bench.measured_traffic("c2", 4, str(tmp_path)) is None and bench.measured_traffic("c3", 2, str(tmp_path)) is None
+    (src / "k_plasma.hip").write_text("// another comment\nint kernel;\n")
+    assert bench.measured_traffic("c2", 2, str(tmp_path)) == 41387494.0
+    (src / "k_plasma.hip").write_text("int kernel = 1;\n")
+    assert bench.measured_traffic("c2", 2, str(tmp_path)) is None
