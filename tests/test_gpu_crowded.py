@@ -1,8 +1,8 @@
 """Parity where radial cells hold more particles than one deposit wave takes.
 
-A wave deposits at most 1024 particles of a cell; the further chunks of a
-crowded cell are deposited by overflow waves into overflow partial rows that
-every consumer adds in row order (the charge deposit and the slice sources,
+A crowded cell is deposited in chunks of 1024 particles, each shared by the
+four waves of a workgroup; the chunks after the first go to overflow partial
+rows that every consumer adds in row order (the charge deposit and the slice sources,
 the current deposit and the iteration sources, and the fine-grained combine
 kernels).  The small C-style decks elsewhere never crowd a cell that much, so
 this deck puts 3000 particles in every radial cell (three chunks: 1024, 1024,

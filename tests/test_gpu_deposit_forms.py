@@ -1,5 +1,5 @@
 """The current deposit's two accumulation forms (include/qpad_hip.h,
-qpad_launch_shape.dep_mfma): the wave reduce-scatter and the FP64 matrix-core
+qpad_launch_shape.dep_mfma): lane accumulators and the FP64 matrix-core
 GEMM add the same per-particle terms (amjdeposit_robust_part2d /
 amjdeposit_std_part2d, part2d_class.f03:877-960) in different orders.  Each
 form matches the oracle slice by slice, the two agree to rounding over a
